@@ -442,12 +442,8 @@ int materialize(InType in, const Opnd &o, int64_t R, int64_t K, int64_t batch, u
     const size_t esz = in_size(in);
     const int64_t ld = round_up64(std::max<int64_t>(K, 1), 16 / (int64_t)esz);
     const int64_t nb = (batch > 1 && o.bs != 0) ? batch : 1;
-    for (int64_t z = 0; z < nb; ++z) {
-        const uint8_t *src = (const uint8_t *)o.p + z * o.bs * (int64_t)esz;
-        hipError_t e = launch_pack(in, src, o.rs, o.ks, R, K, dst + z * R * ld * (int64_t)esz, ld,
-                                   tl_stream);
-        if (e != hipSuccess) return hip_fail(e, "pack");
-    }
+    hipError_t e = launch_pack(in, o.p, o.rs, o.ks, o.bs, R, K, dst, ld, nb, tl_stream);
+    if (e != hipSuccess) return hip_fail(e, "pack");
     *out = Opnd{dst, ld, 1, nb > 1 ? R * ld : 0};
     return GK_OK;
 }
@@ -1670,7 +1666,7 @@ int prepack_any(InType in, const void *b, ptrdiff_t rsb, ptrdiff_t csb, size_t k
             return fail(GK_ERR_NOMEM, "gemmkit: prepacked RHS allocation of %zu bytes failed", bytes);
         }
         // Row j of the buffer is column j of B.
-        e = launch_pack(in, b, csb, rsb, (int64_t)n, (int64_t)k, p->buf, p->ld, tl_stream);
+        e = launch_pack(in, b, csb, rsb, 0, (int64_t)n, (int64_t)k, p->buf, p->ld, 1, tl_stream);
         if (e == hipSuccess) e = hipStreamSynchronize(tl_stream);
         if (e != hipSuccess) {
             (void)hipFree(p->buf);
@@ -1817,7 +1813,7 @@ int prepack_lhs_any(InType in, const void *a, ptrdiff_t rsa, ptrdiff_t csa, size
             delete p;
             return fail(GK_ERR_NOMEM, "gemmkit: prepacked LHS allocation of %zu bytes failed", bytes);
         }
-        e = launch_pack(in, a, rsa, csa, (int64_t)m, (int64_t)k, p->buf, p->ld, tl_stream);
+        e = launch_pack(in, a, rsa, csa, 0, (int64_t)m, (int64_t)k, p->buf, p->ld, 1, tl_stream);
         if (e == hipSuccess) e = hipStreamSynchronize(tl_stream);
         if (e != hipSuccess) {
             (void)hipFree(p->buf);

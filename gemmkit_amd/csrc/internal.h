@@ -162,10 +162,13 @@ constexpr int64_t kSkinnyLdsMax = 128 * 1024;
 int64_t skinny_lds_bytes(InType in, int64_t K, int nvec);
 hipError_t launch_skinny(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
 
-// Pack a strided rows x K operand into a k-contiguous buffer with row stride
-// ld (>= K, ld*esize a multiple of 16); columns [K, ld) are zero-filled.
-hipError_t launch_pack(InType in, const void *src, int64_t rs, int64_t cs, int64_t rows,
-                       int64_t K, void *dst, int64_t ld, hipStream_t stream);
+// Pack `batch` (at most kMaxGridZ) strided rows x K operands, bs elements apart,
+// into a k-contiguous buffer with row stride ld (>= K, ld*esize a multiple of
+// 16; dst 16-byte aligned), element z at dst + z*rows*ld; columns [K, ld) are
+// zero-filled.
+hipError_t launch_pack(InType in, const void *src, int64_t rs, int64_t cs, int64_t bs,
+                       int64_t rows, int64_t K, void *dst, int64_t ld, int64_t batch,
+                       hipStream_t stream);
 
 // C <- beta*C for the degenerate k == 0 / alpha == 0 cases (scale_c_int,
 // src/dispatch/int.rs:150-163, and its float twin src/dispatch.rs:484-497).
