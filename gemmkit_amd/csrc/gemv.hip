@@ -22,6 +22,9 @@
 //     time, 32 KiB per batch, the next batch in flight behind the current.
 //   * gemv_lds: longer rows, more vectors.  The vectors are staged in LDS and
 //     each lane keeps UNROLL chunks per row in flight.
+//   * gemv_cols: a matrix with unit row stride instead (x * W with W row-major),
+//     read in place; sums in the order of whichever kernel above serves the
+//     same shape.
 // Per-lane partial sums of the RPW x NV outputs of a row group are combined by
 // a butterfly over the 64 lanes that halves the number of values each lane
 // carries at every step (V values cost V-1 + log2(64/V) shuffles instead of
@@ -504,6 +507,327 @@ static hipError_t gemv_nv(const GemvArgs &g, const EpiParams &ep, hipStream_t st
     if (g.nvec <= 2) return go_nv<T, E, 2>(g, ep, stream);
     if (g.nvec <= 4) return go_nv<T, E, 4>(g, ep, stream);
     return go_nv<T, E, 8>(g, ep, stream);
+}
+
+// ---------------------------------------------------------- unit row stride
+
+// A 16-byte load at any address (rows of a strided matrix need not be aligned).
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+
+// x[k] of a staged chunk, widened, and the multiply of one matrix chunk row.
+template <InType T>
+struct ColStep;
+
+template <>
+struct ColStep<InType::F32> {
+    static constexpr int EPC = 4;
+    using acc_t = float;
+    using elem_t = uint32_t;
+    // m[e]: EPC consecutive matrix rows at k = e of the chunk; x: the chunk's EPC
+    // vector elements.  Ascending k, one FMA each: Dot16's order.
+    __device__ __forceinline__ static void mul(const v4i_g (&m)[4], v4i_g x, acc_t (&acc)[4]) {
+        const v4f_g xf = __builtin_bit_cast(v4f_g, x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const v4f_g mf = __builtin_bit_cast(v4f_g, m[e]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(mf[r], xf[e], acc[r]);
+        }
+    }
+};
+
+template <>
+struct ColStep<InType::BF16> {
+    static constexpr int EPC = 8;
+    using acc_t = float;
+    using elem_t = uint16_t;
+    __device__ __forceinline__ static float at(const v4i_g &v, int i) {
+        const uint32_t w = (uint32_t)v[i >> 1];
+        return __uint_as_float((i & 1) ? (w & 0xFFFF0000u) : (w << 16));
+    }
+    __device__ __forceinline__ static void mul(const v4i_g (&m)[8], v4i_g x, acc_t (&acc)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float xe = at(x, e);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) acc[r] = __builtin_fmaf(at(m[e], r), xe, acc[r]);
+        }
+    }
+};
+
+template <>
+struct ColStep<InType::I8> {
+    static constexpr int EPC = 16;
+    using acc_t = int32_t;
+    using elem_t = uint8_t;
+    // 4 x 4 byte transposes bring four k of one matrix row into a word.
+    __device__ __forceinline__ static void mul(const v4i_g (&m)[16], v4i_g x, acc_t (&acc)[16]) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint32_t i0 = m[4 * p][c], i1 = m[4 * p + 1][c];
+                const uint32_t i2 = m[4 * p + 2][c], i3 = m[4 * p + 3][c];
+                const uint32_t t0 = __builtin_amdgcn_perm(i1, i0, 0x05010400u);
+                const uint32_t t1 = __builtin_amdgcn_perm(i1, i0, 0x07030602u);
+                const uint32_t u0 = __builtin_amdgcn_perm(i3, i2, 0x05010400u);
+                const uint32_t u1 = __builtin_amdgcn_perm(i3, i2, 0x07030602u);
+                const uint32_t w[4] = {__builtin_amdgcn_perm(u0, t0, 0x05040100u),
+                                       __builtin_amdgcn_perm(u0, t0, 0x07060302u),
+                                       __builtin_amdgcn_perm(u1, t1, 0x05040100u),
+                                       __builtin_amdgcn_perm(u1, t1, 0x07060302u)};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    acc[4 * c + r] = __builtin_amdgcn_sdot4((int)w[r], x[p], acc[4 * c + r], false);
+            }
+    }
+};
+
+// out[j, r] with a matrix of unit row stride (element (r, p) at r + p*mks, any
+// mks and alignment) and k-contiguous vectors (any alignment).  Bound by
+// streaming the matrix once: bf16 1 x 4096 x 11008 17.1 us (5.3 TB/s with three
+// copies in turn, 20.6 from HBM alone) against 55 with the matrix packed first,
+// f32 30.6 against 96, i8 12.0 against 44.  A lane loads 16 bytes of EPC consecutive matrix
+// rows at one k; eight lanes side by side cover a run of 128 bytes (64-byte runs
+// measured slower), and 64 slots split K by 16-byte chunks: slot s takes chunks
+// s, s + 64, ... -- the chunks lane s of a row kernel multiplies, in the same
+// order, so each slot's partial sum is that lane's.  The slots are then added in
+// the row kernels' butterfly order (32, 16, 8, 4, 2, 1 apart) and, where those
+// run 256 lanes per row (NCL = 4 chunk classes per slot), the four groups in
+// wave order: results equal the row kernels' on a packed copy bit for bit.
+// Slot s of a wave of 8 slots is s*8 + w, so the first three butterfly steps stay
+// inside the wave and the eight waves w of a column group need one exchange: through
+// LDS when one workgroup holds all eight, or (SPLIT, too few columns for the
+// CUs) through global partial sums, a wave per workgroup and class group, that
+// cols_combine adds.
+constexpr int kColLanes = 8;
+
+template <InType T>
+__device__ __forceinline__ typename ColStep<T>::acc_t cols_tree(
+    typename ColStep<T>::acc_t (&v)[kColLanes]) {
+#pragma unroll
+    for (int off = kColLanes / 2; off >= 1; off >>= 1)
+#pragma unroll
+        for (int w = 0; w < off; ++w) v[w] += v[w + off];
+    return v[0];
+}
+
+template <InType T, EpiKind E, int NV, int NCL, int UNR, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 : kColLanes * 64) void gemv_cols(const GemvArgs g,
+                                                                       const EpiParams ep) {
+    using St = ColStep<T>;
+    using acc_t = typename St::acc_t;
+    using elem_t = typename St::elem_t;
+    constexpr int EPC = St::EPC, COLS = kColLanes * EPC;
+    __shared__ acc_t part[SPLIT ? 1 : NCL * NV][SPLIT ? 1 : kColLanes][SPLIT ? 1 : COLS];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t zb = blockIdx.y;
+    const elem_t *mat = (const elem_t *)g.mat + zb * g.bsm;
+    const elem_t *vec = (const elem_t *)g.vec + zb * g.bsv;
+    // SPLIT: workgroup = (column group, class group, wave), waves fastest.
+    const int64_t blk = SPLIT ? blockIdx.x / (NCL * kColLanes) : blockIdx.x;
+    const int wave = SPLIT ? (int)(blockIdx.x % kColLanes)
+                           : __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q0 = SPLIT ? (int)(blockIdx.x / kColLanes) % NCL : 0;
+    const int cl = lane % kColLanes, slot = (lane / kColLanes) * kColLanes + wave;
+    // The last column group's lanes start EPC rows before R at the latest (so
+    // every load stays inside the matrix; the caller ensures R >= EPC); the
+    // rows below their own range are another lane's to store.
+    const int64_t rl = blk * COLS + cl * EPC;
+    const int64_t r0 = rl + EPC <= g.R ? rl : g.R - EPC;
+    constexpr int64_t STEP = 64 * NCL;
+    const int64_t nfull = (int64_t)g.K / EPC;  // whole chunks (at least one: the caller's minimum K)
+
+    auto load = [&](int64_t ch, v4i_g (&m)[EPC], v4i_g (&x)[NV]) {
+        const elem_t *p = mat + r0 + ch * EPC * g.mks;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            x[j] = *(const v4i_any *)(vec + (j < g.nvec ? j : 0) * g.vld + ch * EPC);
+#pragma unroll
+        for (int e = 0; e < EPC; ++e)
+            m[e] = *(const v4i_any *)(p + e * g.mks);
+    };
+    for (int q = q0; q < (SPLIT ? q0 + 1 : NCL); ++q) {
+        acc_t acc[NV][EPC] = {};
+        int64_t ch = slot + 64 * q;
+        // All loads of a batch are issued before any is used (the scheduler
+        // would otherwise sink them to their uses to save registers); chunks
+        // past the end load the last one again and are left out.
+        for (int64_t c0 = 64 * q; c0 < nfull; c0 += STEP * UNR, ch += STEP * UNR) {
+            v4i_g m[UNR][EPC], x[UNR][NV];
+#pragma unroll
+            for (int u = 0; u < UNR; ++u) {
+                const int64_t c = ch + STEP * u;
+                load(c < nfull ? c : nfull - 1, m[u], x[u]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < UNR; ++u)
+                if (ch + STEP * u < nfull) {
+#pragma unroll
+                    for (int j = 0; j < NV; ++j) St::mul(m[u], x[u][j], acc[j]);
+                }
+        }
+        if (nfull * EPC < g.K && nfull % STEP == slot + 64 * q) {  // the last chunk, zeros past K
+            v4i_g m[EPC];
+#pragma unroll
+            for (int e = 0; e < EPC; ++e) {
+                m[e] = v4i_g{0, 0, 0, 0};
+                if (nfull * EPC + e < g.K)
+                    m[e] = *(const v4i_any *)(mat + r0 + (nfull * EPC + e) * g.mks);
+            }
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const elem_t *p = vec + (j < g.nvec ? j : 0) * g.vld + nfull * EPC;
+                elem_t v[EPC];
+#pragma unroll
+                for (int e = 0; e < EPC; ++e) v[e] = nfull * EPC + e < g.K ? p[e] : elem_t(0);
+                v4i_g x;
+                __builtin_memcpy(&x, v, 16);
+                St::mul(m, x, acc[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int r = 0; r < EPC; ++r) {
+#pragma unroll
+                for (int off = 32; off >= kColLanes; off >>= 1)
+                    acc[j][r] += __shfl_xor(acc[j][r], off, 64);
+                if (lane < kColLanes && r0 + r >= rl) {
+                    if constexpr (SPLIT) {
+                        if (j < g.nvec)
+                            ((acc_t *)g.part)[(((zb * NCL + q) * g.nvec + j) * kColLanes + wave) *
+                                                  g.R + r0 + r] = acc[j][r];
+                    } else {
+                        part[q * NV + j][wave][r0 + r - blk * COLS] = acc[j][r];
+                    }
+                }
+            }
+    }
+    if constexpr (!SPLIT) {
+        __syncthreads();
+        for (int o = tid; o < NV * COLS; o += kColLanes * 64) {
+            const int j = o / COLS, c = o % COLS;
+            acc_t sum = acc_t(0);
+#pragma unroll
+            for (int q = 0; q < NCL; ++q) {
+                acc_t v[kColLanes];
+#pragma unroll
+                for (int w = 0; w < kColLanes; ++w) v[w] = part[q * NV + j][w][c];
+                sum = q == 0 ? cols_tree<T>(v) : sum + cols_tree<T>(v);
+            }
+            const int64_t r = blk * COLS + c;
+            if (j < g.nvec && r < g.R) Store<E>::apply(ep, zb, j, (int)r, sum);
+        }
+    }
+}
+
+// Adds SPLIT partial sums [element][class group][vector][wave][row] in the
+// order above, one output per thread.
+template <InType T, EpiKind E, int NCL>
+__global__ __launch_bounds__(64) void cols_combine(const GemvArgs g, const EpiParams ep) {
+    using acc_t = typename ColStep<T>::acc_t;
+    const int64_t r = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    const int j = blockIdx.y;
+    const int64_t zb = blockIdx.z;
+    if (r >= g.R) return;
+    acc_t v[NCL][kColLanes];
+#pragma unroll
+    for (int q = 0; q < NCL; ++q)
+#pragma unroll
+        for (int w = 0; w < kColLanes; ++w)
+            v[q][w] = ((const acc_t *)g.part)[(((zb * NCL + q) * g.nvec + j) * kColLanes + w) *
+                                                  g.R + r];
+    acc_t sum = cols_tree<T>(v[0]);
+#pragma unroll
+    for (int q = 1; q < NCL; ++q) sum = sum + cols_tree<T>(v[q]);
+    Store<E>::apply(ep, zb, j, (int)r, sum);
+}
+
+template <InType T, EpiKind E, int NV, int NCL, int UNR>
+static hipError_t go_cols(const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {
+    constexpr int COLS = kColLanes * ColStep<T>::EPC;
+    const int64_t blocks = ((int64_t)g.R + COLS - 1) / COLS;
+    if (g.part) {
+        hipLaunchKernelGGL((gemv_cols<T, E, NV, NCL, UNR, true>),
+                           dim3((unsigned)(blocks * NCL * kColLanes), (unsigned)g.batch), dim3(64),
+                           0, stream, g, ep);
+        hipLaunchKernelGGL((cols_combine<T, E, NCL>),
+                           dim3((unsigned)((g.R + 63) / 64), (unsigned)g.nvec, (unsigned)g.batch),
+                           dim3(64), 0, stream, g, ep);
+    } else {
+        hipLaunchKernelGGL((gemv_cols<T, E, NV, NCL, UNR, false>),
+                           dim3((unsigned)blocks, (unsigned)g.batch), dim3(kColLanes * 64), 0,
+                           stream, g, ep);
+    }
+    return hipGetLastError();
+}
+
+// The summing order of the row kernel go_nv picks for the same shape: 256
+// lanes per row where that is gemv_wgrow, 64 otherwise (i8 sums have no order).
+static bool cols_wgrow(InType in, int nvec, int64_t K) {
+    const int64_t nch = (K * (int64_t)in_size(in) + 15) / 16;
+    return nch > 512 && (in == InType::F32 ? nvec <= 2 : (in == InType::BF16 && nvec == 1));
+}
+
+// Chunks per slot in one batch of loads: 16 matrix loads (64 registers) of a
+// lane in flight, i8 32 (a chunk of i8 is 16 loads), half with more vectors.
+constexpr int cols_unroll(InType in, int nv) {
+    return (in == InType::F32 ? 4 : 2) / (nv <= 2 ? 1 : 2);
+}
+
+template <InType T, EpiKind E, int NV>
+static hipError_t cols_nv(const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {
+    constexpr int UNR = cols_unroll(T, NV);
+    if constexpr (T == InType::F32 ? NV <= 2 : (T == InType::BF16 && NV == 1)) {
+        if (cols_wgrow(T, g.nvec, g.K)) return go_cols<T, E, NV, 4, UNR>(g, ep, stream);
+    }
+    return go_cols<T, E, NV, 1, UNR>(g, ep, stream);
+}
+
+template <InType T, EpiKind E>
+static hipError_t gemv_cols_nv(const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {
+    if (g.nvec <= 1) return cols_nv<T, E, 1>(g, ep, stream);
+    if (g.nvec <= 2) return cols_nv<T, E, 2>(g, ep, stream);
+    return cols_nv<T, E, 4>(g, ep, stream);
+}
+
+// K is split over workgroups when a slot has more than one batch of loads and
+// the column groups are few for the CUs: 1 x 4096 x 4096 (64 groups) 10.0 against
+// 12.4 us in one workgroup per group, x 1024 (16 groups) 8.1 against 11.5, i8
+// x 11008 (86) 14.7 against 17.9; bf16 x 11008 (172) 18.3 against 17.1 and 1 x
+// 1024 x 16384 (256, one batch) 10.4 against 8.5 stay whole.  With four class
+// groups there are four times as many waves to spread, and it pays up to two
+// groups per CU (f32 1 x 4096 x 11008, 344 groups: 30.6 against 33.1 us).
+int64_t gemv_cols_part_bytes(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus) {
+    const int64_t epc = 16 / (int64_t)in_size(in), cols = kColLanes * epc;
+    const int ncl = cols_wgrow(in, nvec, K) ? 4 : 1;
+    if (K / epc <= 64 * cols_unroll(in, nvec)) return 0;
+    if ((R + cols - 1) / cols * batch > (int64_t)(cus > 0 ? cus : 256) * ncl / 2) return 0;
+    return ncl * batch * nvec * kColLanes * R * 4;
+}
+
+hipError_t launch_gemv_cols(InType in, const GemvArgs &g, const EpiParams &ep,
+                            hipStream_t stream) {
+    if (g.nvec < 1 || g.nvec > kGemvColsMaxVec || g.R < 16 / (int)in_size(in) || g.ld != 1 || g.batch < 1 ||
+        g.batch > kMaxGridZ)
+        return hipErrorInvalidValue;
+    switch (in) {
+    case InType::I8:
+        if (ep.kind == EpiKind::I32) return gemv_cols_nv<InType::I8, EpiKind::I32>(g, ep, stream);
+        if (ep.kind == EpiKind::Q8) return gemv_cols_nv<InType::I8, EpiKind::Q8>(g, ep, stream);
+        break;
+    case InType::F32:
+        if (ep.kind == EpiKind::F32) return gemv_cols_nv<InType::F32, EpiKind::F32>(g, ep, stream);
+        break;
+    case InType::BF16:
+        if (ep.kind == EpiKind::F32) return gemv_cols_nv<InType::BF16, EpiKind::F32>(g, ep, stream);
+        if (ep.kind == EpiKind::BF16)
+            return gemv_cols_nv<InType::BF16, EpiKind::BF16>(g, ep, stream);
+        break;
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_gemv(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {

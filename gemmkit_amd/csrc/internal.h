@@ -134,6 +134,8 @@ struct GemvArgs {
     int32_t cus;           // compute units of the device (persistent grid size)
     int32_t batch;         // batch elements (grid y), at most kMaxGridZ
     int64_t bsm, bsv;      // batch strides of mat and vec in elements
+    int64_t mks;           // k stride of mat: 1, or any with ld == 1 (launch_gemv_cols only)
+    void *part;            // gemv_cols_part_bytes() of scratch, or nullptr (launch_gemv_cols only)
     // Output element (vector j, matrix row r) of batch element z is stored as
     // the epilogue's (row j, column r) of element z: at c + z*bsc + j*rsc +
     // r*csc of the EpiParams.  Each element's arithmetic does not depend on
@@ -155,6 +157,15 @@ hipError_t launch_small_f32(const SmallArgs &g, const EpiParams &ep, hipStream_t
 // skinny and GEMV kernels).
 constexpr int64_t kMaxGridZ = 65535;
 hipError_t launch_gemv(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
+
+// The same for a matrix of unit row stride (g.ld == 1, k stride g.mks) with at
+// least 16 bytes of rows, and at most kGemvColsMaxVec k-contiguous vectors,
+// both read in place with any alignment; bit-identical to launch_gemv on packed
+// operands.  Few columns run K split over workgroups through g.part, which
+// must hold gemv_cols_part_bytes() (0: not split).
+constexpr int kGemvColsMaxVec = 4;
+int64_t gemv_cols_part_bytes(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus);
+hipError_t launch_gemv_cols(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
 
 // Matrix-core skinny route (1..16 vectors): the vectors are staged in LDS,
 // which must hold skinny_lds_bytes() <= kSkinnyLdsMax (a CU has 160 KiB).
