@@ -1064,21 +1064,34 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         const int64_t kc = round_up64((k + splits - 1) / splits, 64 / (int64_t)esz);
         splits = (int)((k + kc - 1) / kc);
     }
-    // Small f32 products that split K (too few 64 x 64 tiles for the CUs)
-    // run in one launch instead: a workgroup per 32 x 32 block with K split
-    // over its 16 waves, operands read in place (no pack, no reduction
-    // launch), when each wave's share stays short -- at most 256 k-pairs of
-    // matrix-core work per round of blocks.  By the element shape only, so a
-    // batched element takes the route of its standalone product.
-    if (in == InType::F32 && splits > 1 && small_f32_enabled()) {
+    // f32 routes, operands read in place (no pack), by the element shape only so
+    // that a batched element takes the route of its standalone product:
+    //  * small_f32: products that would split K (too few 64 x 64 tiles for the
+    //    CUs) in one launch, a workgroup per 32 x 32 block with K split over its 16
+    //    waves, when the blocks fit one round of the CUs (512^3: 7.3 us against 13.8
+    //    on f32x, 200 x 150 x 120 5.5 against 7.7) and each wave's share is short;
+    //  * f32x: split into bf16 parts on the bf16 matrix cores, whatever else is
+    //    beyond the streaming kernel's K (2048^3: 88 us against 140 on the f32 tiles;
+    //    1536 x 640 x 167, two rounds of blocks: 15 us against 24 with small_f32).
+    if (in == InType::F32 && !vector_route) {
         const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
         const int64_t blocks = ((M + 31) / 32) * ((N + 31) / 32);
-        if ((blocks + cus - 1) / cus * ((k + 31) / 32) <= 256) {
-            const SmallArgs sa{A.p, Bt.p, A.rs, A.ks, Bt.rs, Bt.ks, A.bs, Bt.bs,
-                               (int32_t)M, (int32_t)N, (int32_t)k, (int32_t)batch};
+        const SmallArgs sa{A.p, Bt.p, A.rs, A.ks, Bt.rs, Bt.ks, A.bs, Bt.bs,
+                           (int32_t)M, (int32_t)N, (int32_t)k, (int32_t)batch};
+        if (splits > 1 && small_f32_enabled() && blocks <= cus &&
+            (k + 31) / 32 <= 256) {
             hipError_t e = launch_small_f32(sa, ep, tl_stream);
             if (e != hipSuccess) return hip_fail(e, "small f32 gemm launch");
             return finish("small f32 gemm");
+        }
+        if (kbytes > kstream_max_kbytes() && f32x_fits(M, N) &&
+            (splits == 1 || (small_f32_enabled() && blocks > cus &&
+                             (blocks + cus - 1) / cus * ((k + 31) / 32) <= 256))) {
+            ep.vec4 = ep.csc == 1 && (M == 1 || ep.rsc % 4 == 0) && (batch <= 1 || bsc % 4 == 0) &&
+                      ((uintptr_t)c % (uintptr_t)16) == 0;
+            hipError_t e = launch_f32x(sa, ep, splits > 1, g_num_cus, tl_stream);
+            if (e != hipSuccess) return hip_fail(e, "f32 gemm launch");
+            return finish("f32 gemm");
         }
     }
     const size_t a_bytes = pack_a ? pack_bytes(in, M, k, batch, A) : 0;

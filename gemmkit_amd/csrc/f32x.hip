@@ -1,0 +1,448 @@
+// f32x.hip -- f32 GEMM on the bf16 matrix cores, at f32 precision: every operand
+// element is split into three bf16 parts and six of the nine products of parts
+// are summed in f32.
+//
+// Replaces the same layers as mma_kernel.h (src/driver.rs:402-944,
+// src/kernel/float.rs:150-281) for f32 products beyond the short contractions of
+// kstream.hip and the small products of small.hip.
+//
+// Why.  CDNA4's f32 matrix rate is 1/16 of its bf16 rate (157 against 2500
+// TFLOP/s), so six bf16 products per f32 product leave 2.6 times the f32 rate.
+// The split loses nothing: a = h + m + l with h = bf16(a), m = bf16(a - h),
+// l = a - h - m is exact (24 significant bits in three times eight, both
+// subtractions exact), the six products hh, hm, mh, mm, hl, lh are exact in f32
+// pairs of 8-bit significands, and the three left out (ml, lm, ll) are below
+// 2^-26 of |a||b| together.  The running sum is rounded six times per 32 k, once
+// per product of parts, where the f32 instructions round it at least 16 times;
+// with HL (the shapes small.hip would serve, whose sixteen partial sums round
+// less) the five small products, 2^-8 of hh, have accumulators of their own and
+// the large sum is rounded once per 32 k.
+// Measured (row-major, against the f32 tiles with B packed first): 2048^3 88.4 us =
+// 194 TFLOP/s against 140.1, relative error 4.9e-7 against 8.1e-7; 1024^3 22 against
+// 35; 488 x 3136 x 2512 75.6 against 102.8.  Bound by the matrix cores at the
+// clock the chip's power limit leaves them: 78 us on zeros.
+//
+// The split needs every part to be a normal bf16 number: |a| below the largest
+// bf16, and 0 or at least 2^-102.  A tile watches for the rest: the smallest
+// nonzero magnitude of each 64-row panel of A and B while it is split, and any
+// accumulator that is not finite (an infinite or NaN input, or one that rounds
+// to an infinite h, always leaves one).  A 64 x 64 block of the output that
+// such a panel or accumulator touches is computed again with the f32
+// instructions from memory.  The blocks are cut at multiples of 64 whatever
+// the tile, so an element's value does not depend on the tile that computed it.
+//
+// Schedule.  One workgroup of two groups of four waves per BM x BN tile; a stage
+// is 32 k, group g multiplies the stages of its parity (every wave of it a
+// quarter of the tile) and the two partial tiles are added at the end.  The
+// groups alternate, one wave of each per SIMD: while one multiplies stage n from
+// fragments in registers, the other reads the fragments of stage n+1 from LDS,
+// splits the elements of stage n+3 (loaded two slots before) into the slot
+// stage n left, and issues the loads of stage n+5; then a barrier, and the roles
+// change.  The matrix cores so always have a wave with nothing else to wait
+// for, and the splitting, the LDS traffic and the memory latency run beside it.
+// (All eight waves doing all of it in turn: 102 us on 2048^3 against 85.)  A K that
+// is no multiple of 32 has its short stage first, outside the loop.
+//
+// Operands are read in place with any strides (no pack): a k-contiguous operand
+// as two 16-byte loads of 8 k of a row per thread, any other as 8 element loads
+// with the lanes along the rows (coalesced when the rows are contiguous).
+// LDS holds, per stage and part, 64-byte rows of 32 k; row r keeps its 16-byte
+// chunk c in slot c ^ ((r >> 2) & 3), which spreads 16 consecutive rows (a
+// fragment read, and the writes of either load form) over distinct banks.
+// v_mfma_f32_16x16x32_bf16 takes B's fragment as its first operand, so
+// register q of lane l is output row l%16, column 4*(l/16) + q of a block: four
+// consecutive columns, one 16-byte store.
+#include "epilogue.h"
+#include "mma_kernel.h"
+
+namespace gk {
+
+typedef float v4f_x __attribute__((ext_vector_type(4)));
+typedef float v4f_xu __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t v4u_x __attribute__((ext_vector_type(4)));
+typedef __bf16 v8bf_x __attribute__((ext_vector_type(8)));
+
+constexpr int kXStage = 32;              // k per stage
+constexpr int kXRow = kXStage * 2;       // LDS bytes of a row of one part
+// 2 * (bits of 2^-102) - 1: see x_watch.
+constexpr uint32_t kXTiny = ((uint32_t)(127 - 102) << 24) - 1;
+
+// Smallest nonzero |a| seen, as 2*|bits| - 1 (a zero becomes the largest).
+__device__ __forceinline__ uint32_t x_watch(uint32_t t, float a) {
+    const uint32_t v = (__float_as_uint(a) << 1) - 1u;
+    return v < t ? v : t;
+}
+
+// The three bf16 parts of 8 consecutive k of a row.  (Forming the differences
+// with v_dot2_f32_bf16, two instructions fewer per pair, doubled the time of a
+// slot: it contends with the other group's MFMAs, plain VALU does not.)
+__device__ __forceinline__ void x_split(const float (&v)[8], v4u_x &h, v4u_x &m, v4u_x &l) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a0 = v[2 * i], a1 = v[2 * i + 1];
+        const uint32_t hp = bf16x2_rne(a0, a1);
+        const float r0 = a0 - __uint_as_float(hp << 16);
+        const float r1 = a1 - __uint_as_float(hp & 0xFFFF0000u);
+        const uint32_t mp = bf16x2_rne(r0, r1);
+        h[i] = hp;
+        m[i] = mp;
+        l[i] = bf16x2_rne(r0 - __uint_as_float(mp << 16), r1 - __uint_as_float(mp & 0xFFFF0000u));
+    }
+}
+
+// AK / BK: the operand is k-contiguous.
+constexpr int kXThreads = 512, kXGroup = 256;
+// HL: the five small products in accumulators of their own.
+template <int BM, int BN, bool AK, bool BK, bool HL>
+__global__ __launch_bounds__(kXThreads)
+__attribute__((amdgpu_waves_per_eu(BM == 64 ? 4 : 2, BM == 64 ? 4 : 2)))
+void f32x_kernel(const SmallArgs g, const EpiParams ep) {
+    constexpr int WTM = BM / 2, WTN = BN / 2;        // a wave's rows and columns
+    constexpr int TM = WTM / 16, TN = WTN / 16;
+    constexpr int IA = BM * 4 / kXGroup, IB = BN * 4 / kXGroup;  // 8-k chunks per thread and stage
+    static_assert(IA >= 1 && IB >= 1 && 64 % WTM == 0 && 64 % WTN == 0, "tile");
+    constexpr int PART = (BM + BN) * kXRow;          // one part of one stage
+    constexpr int BUF = 3 * PART;
+    constexpr int NPA = BM / 64, NPB = BN / 64;
+    static_assert(kXThreads * TM * TN * 2 * 4 <= 3 * BUF, "exchange of the partial tiles");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[3 * BUF];
+    __shared__ int flags[NPA + NPB + NPA * NPB];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1, gt = tid & (kXGroup - 1);
+    const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
+    const int64_t pid = xcd_logical((int64_t)blockIdx.y * gridDim.x + blockIdx.x,
+                                    (int64_t)gridDim.x * gridDim.y);
+    const int64_t zb = pid / gridDim.x;
+    int tm, tn;
+    tile_coords((int)(pid % gridDim.x), tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const float *A = (const float *)g.a + zb * g.bsa;
+    const float *B = (const float *)g.b + zb * g.bsb;
+    if (tid < NPA + NPB + NPA * NPB) flags[tid] = 0;
+
+    // A thread's NC chunks of a stage, IA of A and the others of B: a row and eight
+    // k, chunk c holding k 4c..4c+3 and 16+4c..16+4c+3 (both operands alike, so any
+    // order pairs the right products).  k-contiguous: four threads side by side
+    // read 64 bytes of a row at a time; otherwise the lanes lie along the rows.
+    // Rows past the matrix edge read its last row (their outputs are not stored).
+    constexpr int NC = IA + IB;
+    auto of_a = [](int i) { return i < IA; };
+    auto ks_of = [&](int i) { return of_a(i) ? g.ksa : g.ksb; };
+    auto kc_of = [&](int i) { return of_a(i) ? AK : BK; };
+    auto row_of = [&](int i) {
+        const int c = gt + (of_a(i) ? i : i - IA) * kXGroup;
+        return kc_of(i) ? c / 4 : c % (of_a(i) ? BM : BN);
+    };
+    auto chunk_of = [&](int i) {
+        const int c = gt + (of_a(i) ? i : i - IA) * kXGroup;
+        return kc_of(i) ? c % 4 : c / (of_a(i) ? BM : BN);
+    };
+    const float *src[NC];
+    uint32_t least[NC];    // x_watch
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int r = row_of(i), c = chunk_of(i);
+        const int64_t o = of_a(i) ? (m0 + r < g.M ? m0 + r : g.M - 1) : (n0 + r < g.N ? n0 + r : g.N - 1);
+        src[i] = (of_a(i) ? A + o * g.rsa : B + o * g.rsb) + 4 * c * ks_of(i);
+        least[i] = 0xFFFFFFFFu;
+    }
+    // LDS byte offset of a chunk in a part: rows 64 further down keep their slot
+    // (k-contiguous), chunks two further on flip one bit of it.
+    auto slot_of = [&](int i) {
+        const int r = row_of(i), c = chunk_of(i);
+        return r * kXRow + ((c ^ ((r >> 2) & 3)) * 16);
+    };
+    const int dst_a = slot_of(0), dst_b = BM * kXRow + slot_of(IA);
+    auto dst = [&](int i) {
+        const int n = of_a(i) ? i : i - IA, d = of_a(i) ? dst_a : dst_b;
+        return kc_of(i) ? d + n * 64 * kXRow : d ^ (n * (kXGroup / (of_a(i) ? BM : BN)) * 16);
+    };
+    // Stage t covers k from 32*(t - rag): the whole stages, after the short one
+    // (the last K % 32 k) when there is one.
+    const int rag = g.K % kXStage != 0, whole = g.K / kXStage, stages = whole + rag;
+
+    float raw[NC][8];
+    v4u_x ph[NC], pm[NC], pl[NC];
+    auto load = [&](int i, int t) {  // a whole stage; past the last one, the last again
+        const int64_t ks = ks_of(i);
+        const float *p = src[i] + (int64_t)((t < stages ? t : stages - 1) - rag) * kXStage * ks;
+        if (kc_of(i)) {
+            const v4f_x lo = *(const v4f_xu *)p, hi = *(const v4f_xu *)(p + 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                raw[i][e] = lo[e];
+                raw[i][4 + e] = hi[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) raw[i][e] = p[(e < 4 ? e : e + 12) * ks];
+        }
+    };
+    auto load_short = [&](int i) {  // zeros past K
+        const float *p = src[i] + (int64_t)whole * kXStage * ks_of(i);
+        const int left = g.K - whole * kXStage - 4 * chunk_of(i);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int k = e < 4 ? e : e + 12;
+            raw[i][e] = k < left ? p[k * ks_of(i)] : 0.0f;
+        }
+    };
+    auto split = [&](int i) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) least[i] = x_watch(least[i], raw[i][e]);
+        x_split(raw[i], ph[i], pm[i], pl[i]);
+        // (keeps the splitting in its slot: the compiler sinks it to the writes)
+        asm volatile("" : "+v"(ph[i]), "+v"(pm[i]), "+v"(pl[i]), "+v"(least[i]));
+    };
+    auto put = [&](uint8_t *buf, int i) {
+        *(v4u_x *)(buf + dst(i)) = ph[i];
+        *(v4u_x *)(buf + PART + dst(i)) = pm[i];
+        *(v4u_x *)(buf + 2 * PART + dst(i)) = pl[i];
+    };
+
+    // This lane's fragment offsets: row l%16 of a block, chunk l/16.
+    const int fr = lane & 15, fc = lane >> 4;
+    const int fsw = (fc ^ ((fr >> 2) & 3)) * 16;
+    const int fa = (wm * WTM + fr) * kXRow + fsw, fb = (BM + wn * WTN + fr) * kXRow + fsw;
+    v8bf_x a[3][TM], b[3][TN];
+    // Part q of NC of a stage's fragments.
+    constexpr int NF = 3 * (TM + TN) / NC;
+    static_assert(3 * (TM + TN) % NC == 0, "fragments per chunk");
+    auto frags = [&](const uint8_t *buf, int q) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            const int x = q * NF + f, p = x / (TM + TN), o = x % (TM + TN);
+            const int off = o < TM ? fa + o * 16 * kXRow : fb + (o - TM) * 16 * kXRow;
+            const v8bf_x v = __builtin_bit_cast(v8bf_x, *(const v4u_x *)(buf + p * PART + off));
+            if (o < TM) a[p][o < TM ? o : 0] = v; else b[p][o < TM ? 0 : o - TM] = v;
+        }
+    };
+    v4f_x acc[TM][TN] = {}, low[HL ? TM : 1][HL ? TN : 1] = {};
+    // Smallest products first; the blocks of a step are independent.  From the
+    // third step on, a chunk of the group's next stage is split beside each
+    // step's MFMAs (a wave issues three VALU instructions while one runs).
+    auto mul = [&]() {
+        constexpr int kPart[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    v4f_x &c = HL && s < 5 ? low[HL ? i : 0][HL ? j : 0] : acc[i][j];
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[kPart[s][0]][j],
+                                                                a[kPart[s][1]][i], c, 0, 0, 0);
+                }
+            if (s >= 6 - NC) {
+                split(s - (6 - NC));
+#pragma unroll
+                for (int x = 0; x < TM * TN; ++x) {
+                    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 56 / (TM * TN) + 1, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // Ends a slot: this wave's LDS reads and writes are done, then the barrier
+    // (loads of later stages stay in flight across it).  The scheduling barriers
+    // keep the slot's MFMAs, which touch no memory, from moving past it: the
+    // groups would take turns instead of running side by side.
+    auto slot_end = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Beside the other group's stage n, which was in buffer `at`: reads the
+    // fragments of stage n+1 from the next buffer, writes the parts of stage n+3
+    // into this one and issues the loads of stage n+5, in turns (a wave issues
+    // in order).  Past the last stage it reads and writes LDS that nobody uses.
+    int at = 0;
+    auto next = [&](int o) { return o == 2 * BUF ? 0 : o + BUF; };
+    auto prep = [&](int n) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            frags(lds + next(at), i);
+            __builtin_amdgcn_sched_barrier(0);
+            put(lds + at, i);
+            load(i, n + 5);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // Stages 0 and 2 (group 0) or 1 (group 1) into LDS; group 1's stage 3 split;
+    // group 0's stage 4 loaded.
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        if (grp == 0 && rag) load_short(i); else load(i, grp);
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        split(i);
+        load(i, grp + 2);
+        put(lds + grp * BUF, i);
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        split(i);
+        if (grp == 0) {
+            put(lds + 2 * BUF, i);
+            load(i, 4);
+        }
+    }
+    slot_end();
+    if (grp == 0) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) frags(lds, i);
+    }
+    slot_end();
+    if (grp == 1) {
+        prep(0);
+        at = next(at);
+        slot_end();
+    }
+    for (int n = grp; n < stages; n += 2) {
+        mul();
+        at = next(at);
+        slot_end();
+        if (n + 1 >= stages) break;
+        prep(n + 1);
+        at = next(at);
+        slot_end();
+    }
+
+    if constexpr (HL) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[i][j][q] += low[i][j][q];
+    }
+    // Which 64 x 64 blocks have to be computed again.
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        if (least[i] < kXTiny) atomicOr(&flags[(of_a(i) ? 0 : NPA) + row_of(i) / 64], 1);
+    // The groups exchange halves of their partial tiles: group 0 keeps rows
+    // blocks [0, TM/2) of each wave's part, group 1 the others.
+    constexpr int TH = TM / 2;
+    v4f_x *ex = (v4f_x *)lds;
+#pragma unroll
+    for (int i = 0; i < TH; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            ex[(i * TN + j) * kXThreads + tid] = grp == 0 ? acc[TH + i][j] : acc[i][j];
+    __syncthreads();
+    v4f_x out[TH][TN];
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < TH; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const v4f_x o = ex[(i * TN + j) * kXThreads + (tid ^ kXGroup)];
+            const v4f_x mine = grp == 0 ? acc[i][j] : acc[TH + i][j];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                out[i][j][q] = mine[q] + o[q];
+                odd = odd || (__float_as_uint(out[i][j][q]) & 0x7F800000u) == 0x7F800000u;
+            }
+        }
+    const int ba = wm * WTM / 64, bb = wn * WTN / 64;
+    if (odd) atomicOr(&flags[NPA + NPB + ba * NPB + bb], 1);
+    __syncthreads();
+    const int mw = m0 + wm * WTM + grp * TH * 16, nw = n0 + wn * WTN;
+    if (flags[ba] | flags[NPA + bb] | flags[NPA + NPB + ba * NPB + bb]) {
+        // v_mfma_f32_16x16x4_f32 on operands from memory, ascending k.
+        const float *ar[TH], *br[TN];
+#pragma unroll
+        for (int i = 0; i < TH; ++i) {
+            const int64_t m = mw + 16 * i + fr < g.M ? mw + 16 * i + fr : g.M - 1;
+            ar[i] = A + m * g.rsa;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int64_t n = nw + 16 * j + fr < g.N ? nw + 16 * j + fr : g.N - 1;
+            br[j] = B + n * g.rsb;
+        }
+#pragma unroll
+        for (int i = 0; i < TH; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) out[i][j] = v4f_x{0, 0, 0, 0};
+        for (int64_t k = 0; k < g.K; k += 4) {
+            const int64_t kk = k + fc;
+            float av[TH], bv[TN];
+#pragma unroll
+            for (int i = 0; i < TH; ++i) av[i] = kk < g.K ? ar[i][kk * g.ksa] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bv[j] = kk < g.K ? br[j][kk * g.ksb] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < TH; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    out[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], out[i][j], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TH; ++i) {
+        const int row = mw + 16 * i + fr;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = nw + 16 * j + 4 * fc;
+            if (row >= g.M || col >= g.N) continue;
+            const float v[4] = {out[i][j][0], out[i][j][1], out[i][j][2], out[i][j][3]};
+            float f[4] = {0, 0, 0, 0};
+            if (ep.fused) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int c = col + e < g.N ? col + e : g.N - 1;
+                    f[e] = fused_bias<false>(ep, ep.axis ? c : row);
+                }
+            }
+            store4<EpiKind::F32, float, StPol::Plain>(ep, zb, row, col, g.N, v, nullptr, nullptr, f);
+        }
+    }
+}
+
+template <int BM, int BN, bool HL>
+static hipError_t f32x_go(const SmallArgs &g, const EpiParams &ep, hipStream_t stream) {
+    const int64_t tiles = ((int64_t)(g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    if (tiles * kXThreads > UINT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)tiles, (unsigned)g.batch), block(kXThreads);
+    const bool ak = g.ksa == 1, bk = g.ksb == 1;
+    if (ak && bk)
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, true, true, HL>), grid, block, 0, stream, g, ep);
+    else if (ak)
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, true, false, HL>), grid, block, 0, stream, g, ep);
+    else if (bk)
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, false, true, HL>), grid, block, 0, stream, g, ep);
+    else
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, false, false, HL>), grid, block, 0, stream, g, ep);
+    return hipGetLastError();
+}
+
+bool f32x_fits(int64_t M, int64_t N) {
+    return ((M + 63) / 64) * ((N + 63) / 64) <= (int64_t)UINT32_MAX / kXThreads;
+}
+
+hipError_t launch_f32x(const SmallArgs &g, const EpiParams &ep, bool fine, int cus,
+                       hipStream_t stream) {
+    if (g.M < 1 || g.N < 1 || g.K < 1 || g.batch < 1 || g.batch > kMaxGridZ ||
+        ep.kind != EpiKind::F32)
+        return hipErrorInvalidValue;
+    // 128 x 128 tiles, one per CU, against 64 x 64 ones, two per CU at a time: a round
+    // of large tiles takes about 3.2 times a round of small ones (2048^3: 86 us in
+    // one round against 114 in four; 2048 x 2049 x 2048, whose 272 large tiles take
+    // two rounds: 175 against 145; 1024^3, a quarter of the CUs: 46 against 22).
+    const int64_t c = cus > 0 ? cus : 256;
+    auto rounds = [&](int64_t t) {
+        return (((g.M + t - 1) / t) * ((g.N + t - 1) / t) * g.batch + c - 1) / c;
+    };
+    if (fine) return f32x_go<64, 64, true>(g, ep, stream);
+    if (16 * rounds(128) <= 5 * rounds(64))
+        return f32x_go<128, 128, false>(g, ep, stream);
+    return f32x_go<64, 64, false>(g, ep, stream);
+}
+
+}  // namespace gk

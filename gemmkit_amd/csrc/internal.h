@@ -153,6 +153,15 @@ struct SmallArgs {
 };
 hipError_t launch_small_f32(const SmallArgs &g, const EpiParams &ep, hipStream_t stream);
 
+// f32 products on the bf16 matrix cores (f32x.hip), operands read in place with
+// any strides; outputs do not depend on the tile it picks, but on `fine` (more
+// accumulators, fewer roundings of the sum), which the caller sets by the element
+// shape.
+// f32x_fits: the tiles of an M x N product fit one launch's grid.
+bool f32x_fits(int64_t M, int64_t N);
+hipError_t launch_f32x(const SmallArgs &g, const EpiParams &ep, bool fine, int cus,
+                       hipStream_t stream);
+
 // Batch elements one launch covers (grid z of the tiles, grid y of the
 // skinny and GEMV kernels).
 constexpr int64_t kMaxGridZ = 65535;

@@ -1,0 +1,108 @@
+"""f32 products on the bf16 matrix cores (f32x.hip): f32 precision over layouts,
+ragged sides and K tails, with and without the epilogue's terms; values the
+split cannot represent (infinities, NaN, the largest and the smallest
+magnitudes); and the same bits from either tile, so from a batch and from its
+elements alone."""
+import pytest
+import torch
+
+import gemmkit_amd as gk
+
+pytestmark = pytest.mark.gpu
+
+
+def randn(n, seed, dev):
+    return torch.randn(n, generator=torch.Generator().manual_seed(seed)).to(dev)
+
+
+def strided(x, layout, pad, dev):
+    """(flat tensor, rs, cs) holding x row- or column-major with padded rows."""
+    rows, cols = x.shape
+    if layout == "row":
+        buf = torch.zeros(rows, cols + pad, device=dev)
+        buf[:, :cols] = x
+        return buf.reshape(-1), cols + pad, 1
+    buf = torch.zeros(cols, rows + pad, device=dev)
+    buf[:, :rows] = x.T
+    return buf.reshape(-1), 1, rows + pad
+
+
+# few roundings (products small.hip would serve, K from 128) and many, 64 x 64 and
+# 128 x 128 tiles, sides around 64 and 128, K around the 32-k stages and their
+# alternation between the two groups, one stage more than the ring
+@pytest.mark.parametrize("m,k,n", [(65, 65, 130), (300, 96, 127), (200, 150, 120), (129, 128, 63),
+                                   (700, 333, 650), (1030, 97, 1000), (2049, 160, 2047),
+                                   (1500, 255, 1601), (4100, 128, 1100)])
+@pytest.mark.parametrize("la,lb,pad", [("row", "row", 0), ("row", "col", 3), ("col", "col", 1),
+                                       ("col", "row", 5)])
+def test_precision(dev, m, k, n, la, lb, pad):
+    a, b = randn(m * k, 1, dev).view(m, k), randn(k * n, 2, dev).view(k, n)
+    ab, rsa, csa = strided(a, la, pad, dev)
+    bb, rsb, csb = strided(b, lb, pad, dev)
+    c0, bias = randn(m * n, 3, dev), randn(n, 4, dev)
+    c = c0.clone()
+    gk.gemm_unchecked(m, k, n, 0.75, ab, rsa, csa, bb, rsb, csb, -1.25, c, n, 1)
+    want = 0.75 * (a.double() @ b.double()) - 1.25 * c0.double().view(m, n)
+    # |error| <= roundings * u * sum |terms|: at most 6 per 32 k in each of two
+    # groups' sums, the split's 2^-26 and the four of the epilogue
+    u = 2.0 ** -24
+    terms = 0.75 * (a.abs().double() @ b.abs().double()) + 1.25 * c0.abs().double().view(m, n)
+    roundings = 6 * ((k + 31) // 32) + 6
+    err = (c.view(m, n).double() - want).abs()
+    assert (err <= roundings * u * terms).all()
+    assert err.norm() <= 1e-6 * want.norm()
+    f = torch.zeros(m * n, device=dev)
+    gk.gemm_fused_unchecked(m, k, n, 1.0, ab, rsa, csa, bb, rsb, csb, 0.0, f, n, 1, bias=bias,
+                            bias_dim=gk.BIAS_PER_COL, act=gk.Activation.Relu)
+    p = torch.zeros(m * n, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, ab, rsa, csa, bb, rsb, csb, 0.0, p, n, 1)
+    assert torch.equal(f.view(m, n), torch.relu(p.view(m, n) + bias))
+
+
+def special(m, k, n, seed, dev):
+    """A and B with an infinity, a NaN, the largest f32, subnormals and rows of
+    magnitudes whose split would leave the bf16 range."""
+    a, b = randn(m * k, seed, dev).view(m, k), randn(k * n, seed + 1, dev).view(k, n)
+    a[3, 5] = float("inf")
+    a[m // 2, 7] = float("nan")
+    a[m - 1, k - 1] = 3.4028234e38  # rounds to an infinite bf16
+    b[:, n - 1] *= 1e-25
+    a[20] *= 1e-36                   # parts below the smallest normal bf16
+    a[21] *= 1e-40                   # subnormal
+    a[70, : k // 2] = 0.0
+    b[9, 2] = float("-inf")
+    return a, b
+
+
+@pytest.mark.parametrize("m,k,n", [(300, 100, 200), (200, 150, 120), (1400, 96, 1300)])
+def test_values_outside_the_split(dev, m, k, n):
+    a, b = special(m, k, n, 11, dev)
+    c = torch.zeros(m * n, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, a.view(-1), k, 1, b.reshape(-1), n, 1, 0.0, c, n, 1)
+    got, want = c.view(m, n).double(), a.double() @ b.double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    big = want.abs() > 3.4028234e38  # infinite in f32
+    assert torch.equal(torch.isinf(got), big & ~torch.isnan(want))
+    ok = ~torch.isnan(want) & ~big
+    terms = (a.nan_to_num(0, 0, 0).abs().double() @ b.nan_to_num(0, 0, 0).abs().double())
+    # one rounding per k at most (the f32 instructions), and the subnormal grid
+    bound = (k + 4) * (2.0 ** -24 * terms + 2.0 ** -149)
+    assert ((got - want).abs()[ok] <= bound[ok]).all()
+
+
+@pytest.mark.parametrize("specials", [False, True])
+@pytest.mark.parametrize("batch,m,k,n", [(8, 1000, 96, 1000), (40, 200, 150, 120)])
+def test_batch_equals_standalone(dev, batch, m, k, n, specials):
+    """8 x (1000 x 96 x 1000) fills the CUs with 128 x 128 tiles, one of them
+    takes 64 x 64 ones."""
+    a, b = randn(batch * m * k, 5, dev).view(batch, m, k), randn(batch * k * n, 6, dev).view(batch, k, n)
+    if specials:
+        a[1], b[1] = special(m, k, n, 21, dev)
+        a[batch - 1, 130] *= 1e-37
+    c = torch.zeros(batch * m * n, device=dev)
+    gk.gemm_batched_unchecked(batch, m, k, n, 1.0, a.reshape(-1), k, 1, m * k, b.reshape(-1), n, 1,
+                              k * n, 0.0, c, n, 1, m * n)
+    for z in range(batch):
+        one = torch.zeros(m * n, device=dev)
+        gk.gemm_unchecked(m, k, n, 1.0, a[z].reshape(-1), k, 1, b[z].reshape(-1), n, 1, 0.0, one, n, 1)
+        assert torch.equal(c.view(batch, -1)[z].view(torch.int32), one.view(torch.int32)), z
