@@ -1080,7 +1080,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
                            (int32_t)M, (int32_t)N, (int32_t)k, (int32_t)batch};
         if (splits > 1 && small_f32_enabled() && blocks <= cus &&
             (k + 31) / 32 <= 256) {
-            hipError_t e = launch_small_f32(sa, ep, tl_stream);
+            hipError_t e = launch_small_f32(sa, ep, g_num_cus, tl_stream);
             if (e != hipSuccess) return hip_fail(e, "small f32 gemm launch");
             return finish("small f32 gemm");
         }

@@ -151,7 +151,7 @@ struct SmallArgs {
     int64_t rsa, ksa, rsb, ksb, bsa, bsb;
     int32_t M, N, K, batch;
 };
-hipError_t launch_small_f32(const SmallArgs &g, const EpiParams &ep, hipStream_t stream);
+hipError_t launch_small_f32(const SmallArgs &g, const EpiParams &ep, int cus, hipStream_t stream);
 
 // f32 products on the bf16 matrix cores (f32x.hip), operands read in place with
 // any strides; outputs do not depend on the tile it picks, but on `fine` (more

@@ -105,3 +105,23 @@ def test_negative_strides(dev):
     ref = A @ B
     got = c.cpu().double().reshape(m, n)
     assert ((got - ref).norm() / ref.norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("k", [128, 131, 160, 191, 255, 515])
+@pytest.mark.parametrize("cols", [False, True])
+def test_one_wave_per_block_equals_standalone(dev, k, cols):
+    """A batch with a block for every SIMD (300 x 4 blocks) runs one wave per block:
+    the sixteen ranges' sums in the same order, so the bits of the standalone call."""
+    batch, m, n = 300, 50, 40
+    g = torch.Generator().manual_seed(k)
+    a = torch.randn(batch * m * k, generator=g).to(dev)
+    b = torch.randn(batch * k * n, generator=g).to(dev)
+    rsa, csa, rsb, csb = (1, m, 1, k) if cols else (k, 1, n, 1)
+    c = torch.ones(batch * m * n, device=dev)
+    gk.gemm_batched_unchecked(batch, m, k, n, 0.5, a, rsa, csa, m * k, b, rsb, csb, k * n, 2.0, c,
+                              n, 1, m * n)
+    for z in range(0, batch, 37):
+        one = torch.ones(m * n, device=dev)
+        gk.gemm_unchecked(m, k, n, 0.5, a, rsa, csa, b, rsb, csb, 2.0, one, n, 1, a_off=z * m * k,
+                          b_off=z * k * n)
+        assert torch.equal(c[z * m * n:(z + 1) * m * n].view(torch.int32), one.view(torch.int32))
