@@ -435,17 +435,14 @@ bool canonical(const Opnd &o, int64_t R, int64_t K, size_t esz, int64_t batch) {
 
 int64_t round_up64(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-// Brings an operand into the k-contiguous layout, packing into `dst` when its
-// own strides do not allow it.  Returns the (possibly new) operand.
-int materialize(InType in, const Opnd &o, int64_t R, int64_t K, int64_t batch, uint8_t *dst,
-                Opnd *out) {
-    const size_t esz = in_size(in);
-    const int64_t ld = round_up64(std::max<int64_t>(K, 1), 16 / (int64_t)esz);
-    const int64_t nb = (batch > 1 && o.bs != 0) ? batch : 1;
-    hipError_t e = launch_pack(in, o.p, o.rs, o.ks, o.bs, R, K, dst, ld, nb, tl_stream);
-    if (e != hipSuccess) return hip_fail(e, "pack");
-    *out = Opnd{dst, ld, 1, nb > 1 ? R * ld : 0};
-    return GK_OK;
+// The pack of an operand whose own strides the kernels cannot read, into `dst`;
+// *o becomes the packed operand.
+PackJob pack_job(InType in, Opnd *o, int64_t R, int64_t K, int64_t batch, uint8_t *dst) {
+    const int64_t ld = round_up64(std::max<int64_t>(K, 1), 16 / (int64_t)in_size(in));
+    const int64_t nb = (batch > 1 && o->bs != 0) ? batch : 1;
+    const PackJob j{o->p, o->rs, o->ks, o->bs, R, K, dst, ld, (int32_t)nb, 0, 0, 0, 0};
+    *o = Opnd{dst, ld, 1, nb > 1 ? R * ld : 0};
+    return j;
 }
 
 size_t pack_bytes(InType in, int64_t R, int64_t K, int64_t batch, const Opnd &o) {
@@ -1124,8 +1121,14 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         uint8_t *dst = nullptr;
         int r = region_get(rg, a_bytes + b_bytes + part_bytes, &dst);
         if (r) return r;
-        if (pack_a && (r = materialize(in, A, M, k, batch, dst, &A))) return r;
-        if (pack_b && (r = materialize(in, Bt, N, k, batch, dst + a_bytes, &Bt))) return r;
+        PackJob jobs[2];
+        int nj = 0;
+        if (pack_a) jobs[nj++] = pack_job(in, &A, M, k, batch, dst);
+        if (pack_b) jobs[nj++] = pack_job(in, &Bt, N, k, batch, dst + a_bytes);
+        if (nj > 0) {
+            const hipError_t e = launch_pack(in, jobs, nj, tl_stream);
+            if (e != hipSuccess) return hip_fail(e, "pack");
+        }
         part = dst + a_bytes + b_bytes;
     }
 
@@ -1699,7 +1702,8 @@ int prepack_any(InType in, const void *b, ptrdiff_t rsb, ptrdiff_t csb, size_t k
             return fail(GK_ERR_NOMEM, "gemmkit: prepacked RHS allocation of %zu bytes failed", bytes);
         }
         // Row j of the buffer is column j of B.
-        e = launch_pack(in, b, csb, rsb, 0, (int64_t)n, (int64_t)k, p->buf, p->ld, 1, tl_stream);
+        PackJob job{b, csb, rsb, 0, (int64_t)n, (int64_t)k, p->buf, p->ld, 1, 0, 0, 0, 0};
+        e = launch_pack(in, &job, 1, tl_stream);
         if (e == hipSuccess) e = hipStreamSynchronize(tl_stream);
         if (e != hipSuccess) {
             (void)hipFree(p->buf);
@@ -1846,7 +1850,8 @@ int prepack_lhs_any(InType in, const void *a, ptrdiff_t rsa, ptrdiff_t csa, size
             delete p;
             return fail(GK_ERR_NOMEM, "gemmkit: prepacked LHS allocation of %zu bytes failed", bytes);
         }
-        e = launch_pack(in, a, rsa, csa, 0, (int64_t)m, (int64_t)k, p->buf, p->ld, 1, tl_stream);
+        PackJob job{a, rsa, csa, 0, (int64_t)m, (int64_t)k, p->buf, p->ld, 1, 0, 0, 0, 0};
+        e = launch_pack(in, &job, 1, tl_stream);
         if (e == hipSuccess) e = hipStreamSynchronize(tl_stream);
         if (e != hipSuccess) {
             (void)hipFree(p->buf);

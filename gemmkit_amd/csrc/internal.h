@@ -182,13 +182,20 @@ constexpr int64_t kSkinnyLdsMax = 128 * 1024;
 int64_t skinny_lds_bytes(InType in, int64_t K, int nvec);
 hipError_t launch_skinny(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
 
-// Pack `batch` (at most kMaxGridZ) strided rows x K operands, bs elements apart,
-// into a k-contiguous buffer with row stride ld (>= K, ld*esize a multiple of
-// 16; dst 16-byte aligned), element z at dst + z*rows*ld; columns [K, ld) are
-// zero-filled.
-hipError_t launch_pack(InType in, const void *src, int64_t rs, int64_t cs, int64_t bs,
-                       int64_t rows, int64_t K, void *dst, int64_t ld, int64_t batch,
-                       hipStream_t stream);
+// Pack `batch` (at most kMaxGridZ) strided rows x K operands, element (r, p) of
+// element z at src + z*bs + r*rs + p*cs, into a k-contiguous buffer with row
+// stride ld (>= K, ld*esize a multiple of 16; dst 16-byte aligned), element z at
+// dst + z*rows*ld; columns [K, ld) are zero-filled.
+struct PackJob {
+    const void *src;
+    int64_t rs, cs, bs, rows, K;
+    void *dst;
+    int64_t ld;
+    int32_t batch;
+    int32_t blocks, copy, p0, p1;  // set by launch_pack
+};
+// One or two packs, in one launch where their strides allow it.
+hipError_t launch_pack(InType in, PackJob *jobs, int n, hipStream_t stream);
 
 // C <- beta*C for the degenerate k == 0 / alpha == 0 cases (scale_c_int,
 // src/dispatch/int.rs:150-163, and its float twin src/dispatch.rs:484-497).

@@ -16,6 +16,7 @@
 //                    call vanishes (src/dispatch/float.rs:661-680).
 //   split_reduce     sums the partial products of a split-K matrix-core launch
 //                    and applies the call's epilogue.
+#include <algorithm>
 #include <type_traits>
 
 #include "epilogue.h"
@@ -27,14 +28,19 @@ namespace gk {
 typedef uint32_t v4u_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t v4u_p __attribute__((ext_vector_type(4)));
 
-// Transposes the EPV x EPV elements of a thread (in[i] holds k = i of EPV
-// consecutive rows) into out[j]: EPV consecutive k of row j.
-template <int ESZ>
-__device__ __forceinline__ void transpose_block(const v4u_p (&in)[16 / ESZ],
-                                                v4u_p (&out)[16 / ESZ]) {
+// The words of a block's row: 16 bytes, or 8 for the 8 x 8 block of bytes.
+typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t v2u_p __attribute__((ext_vector_type(2)));
+template <int BYTES> struct PackVec { using any = v4u_any; using vec = v4u_p; };
+template <> struct PackVec<8> { using any = v2u_any; using vec = v2u_p; };
+
+// Transposes the B x B elements of a thread (in[i] holds k = i of B consecutive
+// rows) into out[j]: B consecutive k of row j.
+template <int ESZ, int B, typename V>
+__device__ __forceinline__ void transpose_block(const V (&in)[B], V (&out)[B]) {
     if constexpr (ESZ == 4) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) out[j] = v4u_p{in[0][j], in[1][j], in[2][j], in[3][j]};
+        for (int j = 0; j < 4; ++j) out[j] = V{in[0][j], in[1][j], in[2][j], in[3][j]};
     } else if constexpr (ESZ == 2) {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
@@ -44,9 +50,9 @@ __device__ __forceinline__ void transpose_block(const v4u_p (&in)[16 / ESZ],
                                                   (j & 1) ? 0x07060302u : 0x05040100u);
     } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < B / 4; ++c)
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < B / 4; ++p) {
                 const uint32_t i0 = in[4 * p][c], i1 = in[4 * p + 1][c];
                 const uint32_t i2 = in[4 * p + 2][c], i3 = in[4 * p + 3][c];
                 const uint32_t t0 = __builtin_amdgcn_perm(i1, i0, 0x05010400u);
@@ -62,44 +68,47 @@ __device__ __forceinline__ void transpose_block(const v4u_p (&in)[16 / ESZ],
 }
 
 // Unit row stride (element (r, p) at r + p*cs): the transposing pack.  Bound by
-// memory.  A lane owns a block of EPV rows x EPV k (16 bytes each way) and
-// transposes it in registers, the wave's lanes lie 8 along the rows x 8 along
-// k, so every load instruction reads 8 runs of 128 bytes and every store
-// writes 8 runs of 128 bytes, with no LDS and no barrier, all EPV loads of a
-// lane in flight at once.  bf16 4096 x 4096: 12.0 us (5.6 TB/s read + write, a
-// large copy reaches 5.2) against 18.8 through pack_kernel's LDS tile with its
-// element-wide accesses, 11008 x 4096 33.3 against 41.1, f32 2048 x 2048 8.0
-// against 9.2.
-template <typename T>
-__global__ __launch_bounds__(256) void pack_tr(const T *__restrict__ src, int64_t cs, int64_t bs,
-                                               int64_t rows, int64_t K, T *__restrict__ dst,
-                                               int64_t ld, int64_t dbs, int tiles_r) {
-    constexpr int ESZ = (int)sizeof(T), EPV = 16 / ESZ;
+// memory, by latency below a few MB.  A lane owns a block of B rows x B k and
+// transposes it in registers; the wave's lanes lie 8 along the rows x 8 along
+// k, so every load instruction reads 8 runs of 8*B elements and every store
+// writes as many, with no LDS and no barrier, all B loads of a lane in flight
+// at once.  B fills 16 bytes (runs of 128), or is 8 for an i8 operand too small
+// to give every CU a few waves that way (1712 x 288: FIGI).  bf16 4096 x 4096:
+// 12.0 us (5.6 TB/s read + write, a large copy reaches 5.2) against 18.8
+// through pack_kernel's LDS tile with its element-wide accesses, 11008 x 4096
+// 33.3 against 41.1, f32 2048 x 2048 8.0 against 9.2.
+template <typename T, int B>
+__device__ __forceinline__ void pack_tr(const PackJob &j, int block) {
+    constexpr int ESZ = (int)sizeof(T);
+    using Vec = typename PackVec<B * ESZ>::vec;
+    using Any = typename PackVec<B * ESZ>::any;
+    const T *src = (const T *)j.src + (int64_t)blockIdx.y * j.bs;
+    T *dst = (T *)j.dst + (int64_t)blockIdx.y * j.rows * j.ld;
+    const int64_t cs = j.cs, rows = j.rows, K = j.K, ld = j.ld;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // A workgroup's four waves: 2 along the rows x 2 along k.  The last lanes
-    // along the rows start EPV rows before the end (the caller ensures rows >=
-    // EPV): rows their neighbours also pack, with the same values.
-    int64_t r0 = ((int64_t)(blockIdx.x % tiles_r) * 16 + (wave & 1) * 8 + (lane & 7)) * EPV;
-    const int64_t p0 = ((int64_t)(blockIdx.x / tiles_r) * 16 + (wave >> 1) * 8 + (lane >> 3)) * EPV;
+    // along the rows start B rows before the end (the caller ensures rows >=
+    // B): rows their neighbours also pack, with the same values.
+    int64_t r0 = ((int64_t)(block % j.p0) * 16 + (wave & 1) * 8 + (lane & 7)) * B;
+    const int64_t p0 = ((int64_t)(block / j.p0) * 16 + (wave >> 1) * 8 + (lane >> 3)) * B;
     if (r0 >= rows || p0 >= ld) return;
-    if (r0 + EPV > rows) r0 = rows - EPV;
-    const T *s = src + (int64_t)blockIdx.y * bs + r0 + p0 * cs;
-    dst += (int64_t)blockIdx.y * dbs;
-    v4u_p in[EPV], out[EPV];
-    if (p0 + EPV <= K) {
+    if (r0 + B > rows) r0 = rows - B;
+    const T *s = src + r0 + p0 * cs;
+    Vec in[B], out[B];
+    if (p0 + B <= K) {
 #pragma unroll
-        for (int i = 0; i < EPV; ++i) in[i] = *(const v4u_any *)(s + i * cs);
+        for (int i = 0; i < B; ++i) in[i] = *(const Any *)(s + i * cs);
     } else {  // zeros past K
 #pragma unroll
-        for (int i = 0; i < EPV; ++i) {
-            in[i] = v4u_p{0, 0, 0, 0};
-            if (p0 + i < K) in[i] = *(const v4u_any *)(s + i * cs);
+        for (int i = 0; i < B; ++i) {
+            in[i] = Vec{};
+            if (p0 + i < K) in[i] = *(const Any *)(s + i * cs);
         }
     }
-    transpose_block<ESZ>(in, out);
+    transpose_block<ESZ, B>(in, out);
     T *d = dst + r0 * ld + p0;
 #pragma unroll
-    for (int j = 0; j < EPV; ++j) *(v4u_p *)(d + j * ld) = out[j];
+    for (int i = 0; i < B; ++i) *(Vec *)(d + i * ld) = out[i];
 }
 
 // The 16 bytes of v from byte `sh` (0..15) on, zeros behind them.
@@ -125,17 +134,17 @@ __device__ __forceinline__ v4u_p shift_down(v4u_p v, int sh) {
 // i8 777 x 1001: 3.8 us against 4.6 through pack_kernel, 11008 x 4097: 22 against 38.
 constexpr int kCopyChunks = 256, kCopyRows = 4;
 template <typename T>
-__global__ __launch_bounds__(256) void pack_copy(const T *__restrict__ src, int64_t rs, int64_t bs,
-                                                 int64_t rows, int64_t K, T *__restrict__ dst,
-                                                 int64_t ld, int64_t dbs, int llog, int blocks_c) {
+__device__ __forceinline__ void pack_copy(const PackJob &j, int block) {
     constexpr int EPV = 16 / (int)sizeof(T);
-    src += (int64_t)blockIdx.y * bs;
-    dst += (int64_t)blockIdx.y * dbs;
+    const T *src = (const T *)j.src + (int64_t)blockIdx.y * j.bs;
+    T *dst = (T *)j.dst + (int64_t)blockIdx.y * j.rows * j.ld;
+    const int64_t rs = j.rs, rows = j.rows, K = j.K, ld = j.ld;
+    const int blocks_c = j.p0, llog = j.p1;
     const int lanes = 1 << llog, groups = 256 >> llog;
     const int64_t cpr = ld / EPV;
-    const int64_t c0 = (int64_t)(blockIdx.x % blocks_c) * kCopyChunks;
+    const int64_t c0 = (int64_t)(block % blocks_c) * kCopyChunks;
     const int64_t c1 = c0 + kCopyChunks < cpr ? c0 + kCopyChunks : cpr;
-    const int64_t r0 = (int64_t)(blockIdx.x / blocks_c) * groups * kCopyRows +
+    const int64_t r0 = (int64_t)(block / blocks_c) * groups * kCopyRows +
                        ((int)threadIdx.x >> llog);
     for (int64_t c = c0 + ((int)threadIdx.x & (lanes - 1)); c < c1; c += lanes) {
         const int64_t p = c * EPV < K - EPV ? c * EPV : K - EPV;  // first element loaded
@@ -151,6 +160,22 @@ __global__ __launch_bounds__(256) void pack_copy(const T *__restrict__ src, int6
             const int64_t r = r0 + u * groups;
             if (r < rows) *(v4u_p *)(dst + r * ld + c * EPV) = shift_down(v[u], sh);
         }
+    }
+}
+
+// One or two operands (the two of a product whose K is ragged) in one launch.
+template <typename T>
+__global__ __launch_bounds__(256) void pack_jobs(const PackJob a, const PackJob b) {
+    const bool first = (int)blockIdx.x < a.blocks;
+    const PackJob &j = first ? a : b;
+    const int block = (int)blockIdx.x - (first ? 0 : a.blocks);
+    if ((int)blockIdx.y >= j.batch) return;
+    if (j.copy) {
+        pack_copy<T>(j, block);
+    } else if (sizeof(T) > 1 || j.p1) {
+        pack_tr<T, 16 / (int)sizeof(T)>(j, block);
+    } else {
+        pack_tr<T, sizeof(T) == 1 ? 8 : 16 / (int)sizeof(T)>(j, block);
     }
 }
 
@@ -193,51 +218,67 @@ __global__ __launch_bounds__(256) void pack_kernel(const T *__restrict__ src, in
     }
 }
 
-template <typename T>
-static hipError_t pack_go(const T *src, int64_t rs, int64_t cs, int64_t bs, int64_t rows,
-                          int64_t K, T *dst, int64_t ld, int64_t dbs, int64_t batch,
-                          hipStream_t stream) {
-    constexpr int EPV = 16 / (int)sizeof(T);
-    constexpr int64_t kMaxX = 1 << 24;  // workgroups of 256 in grid x
-    if (cs == 1 && K >= EPV) {
-        const int64_t cpr = ld / EPV;
+// Plans j for pack_jobs; false when its strides or sizes need pack_kernel.
+static bool plan_pack(PackJob &j, int64_t epv) {
+    constexpr int64_t kMaxX = 1 << 23;  // workgroups of 256 in grid x, two jobs together
+    int64_t blocks;
+    if (j.cs == 1 && j.K >= epv) {
+        const int64_t cpr = j.ld / epv;
         int llog = 0;
         while (llog < 6 && (1 << llog) < cpr) ++llog;
         const int64_t rpb = (int64_t)(256 >> llog) * kCopyRows;
-        const int64_t bc = (cpr + kCopyChunks - 1) / kCopyChunks, br = (rows + rpb - 1) / rpb;
-        if (bc * br < kMaxX) {
-            hipLaunchKernelGGL(pack_copy<T>, dim3((unsigned)(bc * br), (unsigned)batch), dim3(256),
-                               0, stream, src, rs, bs, rows, K, dst, ld, dbs, llog, (int)bc);
-            return hipGetLastError();
-        }
-    } else if (rs == 1 && rows >= EPV) {
-        const int64_t tr = (rows + 16 * EPV - 1) / (16 * EPV), tk = (ld + 16 * EPV - 1) / (16 * EPV);
-        if (tr * tk < kMaxX) {
-            hipLaunchKernelGGL(pack_tr<T>, dim3((unsigned)(tr * tk), (unsigned)batch), dim3(256), 0,
-                               stream, src, cs, bs, rows, K, dst, ld, dbs, (int)tr);
-            return hipGetLastError();
-        }
+        const int64_t bc = (cpr + kCopyChunks - 1) / kCopyChunks;
+        blocks = bc * ((j.rows + rpb - 1) / rpb);
+        j.copy = 1;
+        j.p0 = (int)bc;
+        j.p1 = llog;
+    } else if (j.rs == 1 && j.rows >= epv) {
+        // 16-byte blocks; i8 takes 8 x 8 ones while they leave fewer than about
+        // four waves per CU.
+        j.copy = 0;
+        j.p1 = epv < 16 || (double)j.rows * j.ld * j.batch >= 1024.0 * 64 * 256;
+        const int64_t b = j.p1 ? epv : 8;
+        const int64_t tr = (j.rows + 16 * b - 1) / (16 * b);
+        blocks = tr * ((j.ld + 16 * b - 1) / (16 * b));
+        j.p0 = (int)tr;
+    } else {
+        return false;
     }
-    const dim3 grid((unsigned)((ld + 63) / 64), (unsigned)((rows + 63) / 64), (unsigned)batch);
-    hipLaunchKernelGGL(pack_kernel<T>, grid, dim3(256), 0, stream, src, rs, cs, bs, rows, K, dst,
-                       ld, dbs);
+    if (blocks >= kMaxX) return false;
+    j.blocks = (int)blocks;
+    return true;
+}
+
+template <typename T>
+static hipError_t pack_go(PackJob *jobs, int n, hipStream_t stream) {
+    PackJob run[2] = {};
+    int nr = 0;
+    for (int i = 0; i < n; ++i) {
+        PackJob &j = jobs[i];
+        if (plan_pack(j, 16 / (int)sizeof(T))) {
+            run[nr++] = j;
+            continue;
+        }
+        const dim3 grid((unsigned)((j.ld + 63) / 64), (unsigned)((j.rows + 63) / 64),
+                        (unsigned)j.batch);
+        hipLaunchKernelGGL(pack_kernel<T>, grid, dim3(256), 0, stream, (const T *)j.src, j.rs,
+                           j.cs, j.bs, j.rows, j.K, (T *)j.dst, j.ld, j.rows * j.ld);
+    }
+    if (nr > 0)
+        hipLaunchKernelGGL(pack_jobs<T>, dim3((unsigned)(run[0].blocks + run[1].blocks),
+                                              (unsigned)std::max(run[0].batch, run[1].batch)),
+                           dim3(256), 0, stream, run[0], run[1]);
     return hipGetLastError();
 }
 
-hipError_t launch_pack(InType in, const void *src, int64_t rs, int64_t cs, int64_t bs,
-                       int64_t rows, int64_t K, void *dst, int64_t ld, int64_t batch,
-                       hipStream_t stream) {
-    if (batch < 1 || batch > kMaxGridZ) return hipErrorInvalidValue;
+hipError_t launch_pack(InType in, PackJob *jobs, int n, hipStream_t stream) {
+    if (n < 1 || n > 2) return hipErrorInvalidValue;
+    for (int i = 0; i < n; ++i)
+        if (jobs[i].batch < 1 || jobs[i].batch > kMaxGridZ) return hipErrorInvalidValue;
     switch (in_size(in)) {
-    case 1:
-        return pack_go((const uint8_t *)src, rs, cs, bs, rows, K, (uint8_t *)dst, ld, rows * ld,
-                       batch, stream);
-    case 2:
-        return pack_go((const uint16_t *)src, rs, cs, bs, rows, K, (uint16_t *)dst, ld, rows * ld,
-                       batch, stream);
-    default:
-        return pack_go((const uint32_t *)src, rs, cs, bs, rows, K, (uint32_t *)dst, ld, rows * ld,
-                       batch, stream);
+    case 1: return pack_go<uint8_t>(jobs, n, stream);
+    case 2: return pack_go<uint16_t>(jobs, n, stream);
+    default: return pack_go<uint32_t>(jobs, n, stream);
     }
 }
 
