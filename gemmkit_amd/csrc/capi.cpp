@@ -975,8 +975,7 @@ int run_product(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k,
     fe.rsc = rsc;
     fe.csc = csc;
     fe.bsc = bsc;
-    fe.vec4 = csc == 1 && (m == 1 || rsc % 4 == 0) && (batch <= 1 || bsc % 4 == 0) &&
-              ((uintptr_t)c % (uintptr_t)(4 * osz)) == 0;
+    fe.vec4 = csc == 1;
     hipError_t e = launch_split_reduce(in, base, 1, m, n, batch, fe, tl_stream);
     if (e != hipSuccess) return hip_fail(e, "k-slice epilogue launch");
     return finish("mfma gemm (K sliced)");
@@ -1084,8 +1083,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         if (kbytes > kstream_max_kbytes() && f32x_fits(M, N) &&
             (splits == 1 || (small_f32_enabled() && blocks > cus &&
                              (blocks + cus - 1) / cus * ((k + 31) / 32) <= 256))) {
-            ep.vec4 = ep.csc == 1 && (M == 1 || ep.rsc % 4 == 0) && (batch <= 1 || bsc % 4 == 0) &&
-                      ((uintptr_t)c % (uintptr_t)16) == 0;
+            ep.vec4 = ep.csc == 1;
             hipError_t e = launch_f32x(sa, ep, splits > 1, g_num_cus, tl_stream);
             if (e != hipSuccess) return hip_fail(e, "f32 gemm launch");
             return finish("f32 gemm");
@@ -1162,11 +1160,8 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         return finish(skinny_ok ? "skinny" : "gemv");
     }
 
-    // Whole 4-element output chunks can go out as one vector access when C is
-    // unit-stride along the kernel's columns and every chunk start is aligned.
     const int64_t osz = out_size(ep.kind);
-    ep.vec4 = ep.csc == 1 && (M == 1 || ep.rsc % 4 == 0) && (batch <= 1 || bsc % 4 == 0) &&
-              ((uintptr_t)c % (uintptr_t)(4 * osz)) == 0;
+    ep.vec4 = ep.csc == 1;
     MmaArgs args{};
     args.a = A.p;
     args.b = Bt.p;
@@ -1193,7 +1188,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         pe.rsc = N;
         pe.csc = 1;
         pe.bsc = M * N;
-        pe.vec4 = N % 4 == 0;
+        pe.vec4 = 1;
         for (int64_t z0 = 0; z0 < batch; z0 += zchunk) {
             MmaArgs az = args;
             az.batch = (int32_t)std::min(zchunk, batch - z0);

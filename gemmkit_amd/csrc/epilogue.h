@@ -178,10 +178,11 @@ constexpr StPol q8_pol(StPol p) { return p == StPol::WT ? StPol::WT : StPol::Pla
 template <StPol P, typename V>
 __device__ __forceinline__ void st_out(V *p, V v) {
     static_assert(sizeof(V) == 16 || sizeof(V) == 4, "16-byte chunks or 4-byte words");
+    typedef V any_t __attribute__((aligned(1)));  // p need not be aligned
     if constexpr (P == StPol::Plain) {
-        *p = v;
+        *(any_t *)p = v;
     } else if constexpr (P == StPol::NT) {
-        __builtin_nontemporal_store(v, p);
+        __builtin_nontemporal_store(v, (any_t *)p);
     } else if constexpr (sizeof(V) == 16) {
         if constexpr (P == StPol::WT)
             asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
@@ -195,10 +196,16 @@ __device__ __forceinline__ void st_out(V *p, V v) {
     }
 }
 
+// A 4-element chunk of C (16, 8 or 4 bytes) at any element address: one vector
+// access, aligned or not.
+typedef int v4i_any4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float v4f_any4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t v2u_any2 __attribute__((ext_vector_type(2), aligned(2)));
+
 // Four consecutive output columns (col .. col+3) of one row, from the
-// LDS-staged accumulators.  `vec` (uniform) says C is unit-stride along columns
-// and 4-element aligned, so whole chunks take one vector access; otherwise, and
-// for chunks that straddle the matrix edge, each element is stored alone.
+// LDS-staged accumulators.  Where C is unit-stride along columns (ep.vec4,
+// uniform) whole chunks take one vector access; otherwise, and for chunks that
+// straddle the matrix edge, each element is stored alone.
 // Requantization uses the caller's per-element channel scale and bias (qs,
 // qb): the f32 path for all four, its tie correction for every lane of the
 // wave when any lane's product sits on a half, and the exact integer path for
@@ -256,7 +263,7 @@ __device__ __forceinline__ void store4(const EpiParams &ep, int64_t z, int row, 
         v4i_e o;
         for (int e = 0; e < 4; ++e) o[e] = (int32_t)((uint32_t)ep.alpha_i * (uint32_t)v[e]);
         if (ep.beta_i != 0) {
-            v4i_e old = *c;
+            v4i_e old = *(const v4i_any4 *)c;
             for (int e = 0; e < 4; ++e)
                 o[e] = (int32_t)((ep.beta_i == 1 ? (uint32_t)old[e]
                                                  : (uint32_t)ep.beta_i * (uint32_t)old[e]) +
@@ -269,7 +276,7 @@ __device__ __forceinline__ void store4(const EpiParams &ep, int64_t z, int row, 
         v4f_e o;
         for (int e = 0; e < 4; ++e) o[e] = ep.alpha_f * v[e];
         if (ep.beta_f != 0.0f) {
-            v4f_e old = *c;
+            v4f_e old = *(const v4f_any4 *)c;
             for (int e = 0; e < 4; ++e)
                 o[e] = ep.beta_f == 1.0f ? old[e] + o[e] : __builtin_fmaf(ep.beta_f, old[e], o[e]);
         }
@@ -283,7 +290,7 @@ __device__ __forceinline__ void store4(const EpiParams &ep, int64_t z, int row, 
         float f[4];
         for (int e = 0; e < 4; ++e) f[e] = ep.alpha_f * v[e];
         if (ep.beta_f != 0.0f) {
-            v2u_e old = *c;
+            v2u_e old = *(const v2u_any2 *)c;
             for (int e = 0; e < 4; ++e) {
                 float w = bf16_widen((uint16_t)(old[e >> 1] >> (16 * (e & 1))));
                 f[e] = ep.beta_f == 1.0f ? w + f[e] : __builtin_fmaf(ep.beta_f, w, f[e]);
@@ -295,7 +302,7 @@ __device__ __forceinline__ void store4(const EpiParams &ep, int64_t z, int row, 
         v2u_e o;
         o[0] = bf16x2_rne(f[0], f[1]);
         o[1] = bf16x2_rne(f[2], f[3]);
-        __builtin_nontemporal_store(o, c);
+        __builtin_nontemporal_store(o, (v2u_any2 *)c);
     } else {
         const uint32_t word = (uint32_t)(q[0] & 0xFF) | ((uint32_t)(q[1] & 0xFF) << 8) |
                               ((uint32_t)(q[2] & 0xFF) << 16) | ((uint32_t)q[3] << 24);
@@ -364,7 +371,7 @@ __device__ __forceinline__ uint32_t requant_pack4(const EpiParams &ep, const int
 }
 
 // store4 for a chunk wholly inside the matrix with C unit-stride along
-// columns and 4-element aligned (ep.vec4), at the address p of its first
+// columns (ep.vec4), at the address p of its first
 // element, which the caller steps from chunk to chunk instead of forming it
 // from (row, col) with 64-bit multiplies.  alpha = 1 skips the i32 multiplies;
 // requantized chunks take requant_pack4 (`tame` as there).  Results equal
@@ -383,7 +390,7 @@ __device__ __forceinline__ void store4_at(const EpiParams &ep, void *p, const A 
         if (ep.alpha_i != 1)
             for (int e = 0; e < 4; ++e) o[e] = (int32_t)((uint32_t)ep.alpha_i * (uint32_t)o[e]);
         if (ep.beta_i != 0) {
-            v4i_e old = *c;
+            v4i_e old = *(const v4i_any4 *)c;
             for (int e = 0; e < 4; ++e)
                 o[e] = (int32_t)((ep.beta_i == 1 ? (uint32_t)old[e]
                                                  : (uint32_t)ep.beta_i * (uint32_t)old[e]) +
@@ -396,7 +403,7 @@ __device__ __forceinline__ void store4_at(const EpiParams &ep, void *p, const A 
         v4f_e o;
         for (int e = 0; e < 4; ++e) o[e] = ep.alpha_f * v[e];
         if (ep.beta_f != 0.0f) {
-            v4f_e old = *c;
+            v4f_e old = *(const v4f_any4 *)c;
             for (int e = 0; e < 4; ++e)
                 o[e] = ep.beta_f == 1.0f ? old[e] + o[e] : __builtin_fmaf(ep.beta_f, old[e], o[e]);
         }
@@ -410,7 +417,7 @@ __device__ __forceinline__ void store4_at(const EpiParams &ep, void *p, const A 
         float f[4];
         for (int e = 0; e < 4; ++e) f[e] = ep.alpha_f * v[e];
         if (ep.beta_f != 0.0f) {
-            v2u_e old = *c;
+            v2u_e old = *(const v2u_any2 *)c;
             for (int e = 0; e < 4; ++e) {
                 float w = bf16_widen((uint16_t)(old[e >> 1] >> (16 * (e & 1))));
                 f[e] = ep.beta_f == 1.0f ? w + f[e] : __builtin_fmaf(ep.beta_f, w, f[e]);
@@ -422,7 +429,7 @@ __device__ __forceinline__ void store4_at(const EpiParams &ep, void *p, const A 
         v2u_e o;
         o[0] = bf16x2_rne(f[0], f[1]);
         o[1] = bf16x2_rne(f[2], f[3]);
-        __builtin_nontemporal_store(o, c);
+        __builtin_nontemporal_store(o, (v2u_any2 *)c);
     }
 }
 

@@ -36,7 +36,8 @@ struct EpiParams {
     const int32_t *bias;   // per-channel bias or nullptr
     int32_t axis;          // 0: channel = kernel row, 1: channel = kernel column
     int32_t zp, lo, hi;    // zero point and clamp band (ReLU already folded into lo)
-    int32_t vec4;          // C is unit-stride along columns and 4-element aligned
+    int32_t vec4;          // C is unit-stride along columns: whole 4-element chunks go out as
+                           // one vector access, at any alignment
     // fused bias and activation (EpiKind::F32 / BF16, FusedEpi in
     // src/kernel/epilogue.rs:269-330): v <- act(v + fbias[channel]) on the f32
     // value the plain store would write, channel along `axis`; fbias holds f32
