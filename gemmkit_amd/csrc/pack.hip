@@ -73,10 +73,11 @@ __device__ __forceinline__ void transpose_block(const V (&in)[B], V (&out)[B]) {
 // k, so every load instruction reads 8 runs of 8*B elements and every store
 // writes as many, with no LDS and no barrier, all B loads of a lane in flight
 // at once.  B fills 16 bytes (runs of 128), or is 8 for an i8 operand too small
-// to give every CU a few waves that way (1712 x 288: FIGI).  bf16 4096 x 4096:
-// 12.0 us (5.6 TB/s read + write, a large copy reaches 5.2) against 18.8
-// through pack_kernel's LDS tile with its element-wide accesses, 11008 x 4096
-// 33.3 against 41.1, f32 2048 x 2048 8.0 against 9.2.
+// to give every CU a few waves that way (i8 1712 x 288 x 128 with A column-major
+// 7.2 us in all against 8.5).  bf16 4096 x 4096: 12.0 us (5.6 TB/s read + write,
+// a large copy reaches 5.2) against 18.8 through pack_kernel's LDS tile with its
+// element-wide accesses, 11008 x 4096 33.3 against 41.1, f32 2048 x 2048 8.0
+// against 9.2.
 template <typename T, int B>
 __device__ __forceinline__ void pack_tr(const PackJob &j, int block) {
     constexpr int ESZ = (int)sizeof(T);
