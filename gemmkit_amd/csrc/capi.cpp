@@ -852,6 +852,8 @@ constexpr int64_t kSlabMax = int64_t(64) << 20;
 constexpr int64_t kSliceBytes = int64_t(4) << 20;
 // Longest K the wavefront GEMV takes in one launch.
 constexpr int64_t kGemvMaxK = INT32_MAX;
+// Shortest K of the split-bf16 f32 tiles.
+constexpr int64_t kF32xMinK = 128;
 // Shortest row the unit-row-stride GEMV takes: one 16-byte chunk for each of
 // a workgroup's 64 slots.
 constexpr int64_t kGemvColsMinBytes = 1024;
@@ -1080,7 +1082,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
             if (e != hipSuccess) return hip_fail(e, "small f32 gemm launch");
             return finish("small f32 gemm");
         }
-        if (kbytes > kstream_max_kbytes() && f32x_fits(M, N) &&
+        if (k >= kF32xMinK && f32x_fits(M, N) &&
             (splits == 1 || (small_f32_enabled() && blocks > cus &&
                              (blocks + cus - 1) / cus * ((k + 31) / 32) <= 256))) {
             ep.vec4 = ep.csc == 1;

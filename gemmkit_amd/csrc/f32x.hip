@@ -3,8 +3,8 @@
 // are summed in f32.
 //
 // Replaces the same layers as mma_kernel.h (src/driver.rs:402-944,
-// src/kernel/float.rs:150-281) for f32 products beyond the short contractions of
-// kstream.hip and the small products of small.hip.
+// src/kernel/float.rs:150-281) for f32 products with K of 128 or more beyond the
+// small products of small.hip.
 //
 // Why.  CDNA4's f32 matrix rate is 1/16 of its bf16 rate (157 against 2500
 // TFLOP/s), so six bf16 products per f32 product leave 2.6 times the f32 rate.

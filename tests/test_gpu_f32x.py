@@ -27,11 +27,11 @@ def strided(x, layout, pad, dev):
     return buf.reshape(-1), 1, rows + pad
 
 
-# few roundings (products small.hip would serve, K from 128) and many, 64 x 64 and
-# 128 x 128 tiles, sides around 64 and 128, K around the 32-k stages and their
-# alternation between the two groups, one stage more than the ring
-@pytest.mark.parametrize("m,k,n", [(65, 65, 130), (300, 96, 127), (200, 150, 120), (129, 128, 63),
-                                   (700, 333, 650), (1030, 97, 1000), (2049, 160, 2047),
+# few roundings (the blocks of 600 x 700 and 700 x 650, two rounds of the CUs) and
+# many, 64 x 64 and 128 x 128 tiles, sides around 64 and 128, K around the 32-k
+# stages and their alternation between the two groups
+@pytest.mark.parametrize("m,k,n", [(600, 128, 700), (700, 333, 650), (1030, 129, 1000),
+                                   (1300, 131, 900), (1000, 191, 1025), (2049, 160, 2047),
                                    (1500, 255, 1601), (4100, 128, 1100)])
 @pytest.mark.parametrize("la,lb,pad", [("row", "row", 0), ("row", "col", 3), ("col", "col", 1),
                                        ("col", "row", 5)])
@@ -74,7 +74,7 @@ def special(m, k, n, seed, dev):
     return a, b
 
 
-@pytest.mark.parametrize("m,k,n", [(300, 100, 200), (200, 150, 120), (1400, 96, 1300)])
+@pytest.mark.parametrize("m,k,n", [(600, 150, 500), (1400, 130, 1300)])
 def test_values_outside_the_split(dev, m, k, n):
     a, b = special(m, k, n, 11, dev)
     c = torch.zeros(m * n, device=dev)
@@ -91,9 +91,9 @@ def test_values_outside_the_split(dev, m, k, n):
 
 
 @pytest.mark.parametrize("specials", [False, True])
-@pytest.mark.parametrize("batch,m,k,n", [(8, 1000, 96, 1000), (40, 200, 150, 120)])
+@pytest.mark.parametrize("batch,m,k,n", [(8, 1000, 128, 1000), (9, 600, 150, 500)])
 def test_batch_equals_standalone(dev, batch, m, k, n, specials):
-    """8 x (1000 x 96 x 1000) fills the CUs with 128 x 128 tiles, one of them
+    """8 x (1000 x 128 x 1000) fills the CUs with 128 x 128 tiles, one of them
     takes 64 x 64 ones."""
     a, b = randn(batch * m * k, 5, dev).view(batch, m, k), randn(batch * k * n, 6, dev).view(batch, k, n)
     if specials:
