@@ -471,6 +471,7 @@ Tile env_tile(bool *forced) {
     if (!strcmp(s, "256x352w8k128")) return Tile::T256x352w8k128;
     if (!strcmp(s, "256x256w8m16")) return Tile::T256x256w8m16;
     if (!strcmp(s, "256x352w8m16")) return Tile::T256x352w8m16;
+    if (!strcmp(s, "128x256w8m16")) return Tile::T128x256w8m16;
     *forced = false;
     return Tile::T256x256;
 }
@@ -675,7 +676,7 @@ bool tail_split_enabled() {
     return !(s && !strcmp(s, "0"));
 }
 
-// GEMMKIT_HIP_WIDE=0 turns off the one-round 256 x 384 plan.
+// GEMMKIT_HIP_WIDE=0 turns off the one-round plans (256 x 384, 256 x 352, 128 x 256).
 bool wide_round_enabled() {
     const char *s = getenv("GEMMKIT_HIP_WIDE");
     return !(s && !strcmp(s, "0"));
@@ -721,6 +722,19 @@ struct MmaPlan { Tile ta; int32_t pn_a; int64_t na; Tile tb; int32_t pn_b; };
 // 352 rows of B^T with 32-bit offsets from the panel's first row, so they are
 // taken only when those rows plus the K bytes stay below 2^31 (the 256-row
 // tiles are covered by the stride limit the caller enforces by packing).
+// One round of 128 x 256 tiles on 16x16 MFMAs (T128x256w8m16): products with too
+// few 256 x 256 tiles for the CUs whose half tiles fill at least 9/16 of them in
+// one round.  bf16 2048 x 4096 x 4096 (256 tiles) 58.2 us against 72.7 with the
+// 256 x 128 tiles on 32x32 MFMAs the model picks, 2048 x 2048 x 2304 (144 tiles)
+// 29.6 against 35.2, int8 34.2 against 43.6 and 14.0 against 22.2, K of 256 10.2
+// against 13.0 and 9.5 against 10.1; with 128 tiles (2048^3) half the CUs idle: bf16
+// 28.7 against 22.0.
+bool half16_round(int64_t M, int64_t N, int64_t kbytes, InType in) {
+    const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
+    const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256);
+    return m16_allowed(in, kbytes) && 16 * tiles >= 9 * cus && tiles <= cus;
+}
+
 bool wide_fits(const TileCand &c, int64_t ld_b, int64_t kbytes) {
     return panels_fit(1, c.bn, 0, ld_b, kbytes);
 }
@@ -740,6 +754,7 @@ MmaPlan plan_mma(int64_t M, int64_t N, int64_t batch, int64_t kbytes, EpiKind ki
     if (in == InType::BF16 && batch > 1 && !forced) {
         const MmaPlan one = plan_mma(M, N, 1, kbytes, kind, in, ld_b);
         if (one.ta == Tile::T256x256w8m16) return MmaPlan{one.ta, 0, N, one.ta, 0};
+        if (one.ta == Tile::T128x256w8m16) return MmaPlan{one.ta, 0, N, one.ta, 0};
         m16 = false;
     }
     const Tile t = pick_tile(M, N, batch, kbytes, kind, in, &cost, m16);
@@ -750,6 +765,8 @@ MmaPlan plan_mma(int64_t M, int64_t N, int64_t batch, int64_t kbytes, EpiKind ki
         // (a forced wide tile whose rows do not fit is refused at launch)
         return MmaPlan{t, p, N, t, 0};
     }
+    if (batch == 1 && wide_round_enabled() && half16_round(M, N, kbytes, in))
+        return MmaPlan{Tile::T128x256w8m16, 0, N, Tile::T128x256w8m16, 0};
     MmaPlan plan{t, 0, N, t, 0};
     TailSplit ts;
     if (batch == 1 && tail_split_enabled() && plan_tail_split(M, N, kbytes, kind, in, t, cost, &ts)) {
@@ -1068,8 +1085,10 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     //    CUs) in one launch, a workgroup per 32 x 32 block with K split over its 16
     //    waves, when the blocks fit one round of the CUs (512^3: 7.3 us against 13.8
     //    on f32x, 200 x 150 x 120 5.5 against 7.7) and each wave's share is short;
-    //  * f32x: split into bf16 parts on the bf16 matrix cores, whatever else is
-    //    beyond the streaming kernel's K (2048^3: 88 us against 140 on the f32 tiles;
+    //  * f32x: split into bf16 parts on the bf16 matrix cores, whatever else has K
+    //    of 128 or more (below that its four or fewer stages do not pay for its
+    //    start: 951 x 104 x 2368 with k-contiguous operands 15.7 us against 13.9 on
+    //    the f32 tiles; 1500 x 130 x 1500 14.3 against 25.1; 2048^3: 88 us against 140 on the f32 tiles;
     //    1536 x 640 x 167, two rounds of blocks: 15 us against 24 with small_f32).
     if (in == InType::F32 && !vector_route) {
         const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
@@ -1239,7 +1258,18 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     }
     MmaArgs aw = args;
     aw.pn = plan.pn_a;
-    e = launch_mma(in, plan.ta, aw, ep, tl_stream);
+    Tile tile = plan.ta;
+    // A batch of half-tile elements takes whole tiles where they need at most
+    // half the rounds (the same sums: 2 x (2048 x 4096 x 4096) in one round
+    // instead of two).
+    if (tile == Tile::T128x256w8m16 && batch > 1 && !forced) {
+        const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
+        auto rounds = [&](int64_t bm) {
+            return (((M + bm - 1) / bm) * ((N + 255) / 256) * batch + cus - 1) / cus;
+        };
+        if (2 * rounds(256) <= rounds(128)) tile = Tile::T256x256w8m16;
+    }
+    e = launch_mma(in, tile, aw, ep, tl_stream);
     if (e != hipSuccess) return hip_fail(e, "mfma launch");
     return finish("mfma gemm");
 }

@@ -9,7 +9,8 @@ hipError_t launch_mma(InType in, Tile tile, const MmaArgs &args, const EpiParams
     // Tile rows are addressed as unsigned 32-bit offsets from the tile's
     // first row: row strides must be non-negative (the host packs otherwise).
     if (args.lda < 0 || args.ldb < 0) return hipErrorInvalidValue;
-    if (tile == Tile::T256x256w8m16) return launch_mma16(in, args, ep, stream);
+    if (tile == Tile::T256x256w8m16 || tile == Tile::T128x256w8m16)
+        return launch_mma16(in, tile, args, ep, stream);
     if (tile == Tile::T256x352w8m16) return launch_mma16w(in, args, ep, stream);
     switch (in) {
     case InType::I8: return launch_mma_i8(tile, args, ep, stream);

@@ -1,5 +1,10 @@
 // mma16.hip -- the 256 x 256 eight-wave tile on 16x16 matrix-core
-// instructions (v_mfma_i32_16x16x64_i8, v_mfma_f32_16x16x32_bf16).
+// instructions (v_mfma_i32_16x16x64_i8, v_mfma_f32_16x16x32_bf16), and the same on
+// half the rows (BM = 128) for products with too few whole tiles for the CUs.
+// The half tile is LDS-bound (a 64 x 64 wave part reads 16 fragments per 32 MFMAs,
+// the whole tile's 24 per 64) and still beats the 32x32 tiles there: bf16 2048 x 4096
+// x 4096 58.2 us (1.18 PFLOP/s) against 72.7 with 256 x 128 tiles, int8 34.2 (2.01
+// POP/s) against 43.6.
 //
 // Same data path as mma_kernel.h (direct-to-LDS loads of 128-byte stages into
 // a swizzled ring -- here three A slots and two B slots, so a stage's A loads
@@ -47,27 +52,28 @@ struct Mma16x<InType::BF16> {
     }
 };
 
-template <InType T, EpiKind E>
+template <InType T, EpiKind E, int BM>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void mma16_kernel(const MmaArgs args, const EpiParams ep) {
-    constexpr int BM = 256, BN = 256, WN = 4, BK = 128;
+    constexpr int BN = 256, WN = 4, BK = 128;
     constexpr int NWAVES = 8;
-    constexpr int WTM = 128, WTN = 64;
-    constexpr int TM = WTM / 16, TN = WTN / 16;  // 8 x 4 blocks of 16 x 16
-    constexpr int ASTAGE = BM * BK, BSTAGE = BN * BK;  // 32 KiB each
+    constexpr int WTM = BM / 2, WTN = 64;
+    constexpr int TM = WTM / 16, TN = WTN / 16;  // 8 x 4 blocks of 16 x 16 (BM 128: 4 x 4)
+    constexpr int ASTAGE = BM * BK, BSTAGE = BN * BK;  // 32 KiB each (BM 128: A 16)
     constexpr int NSA = 3, NSB = 2;              // A and B ring slots
     constexpr int B_BASE = NSA * ASTAGE;
-    constexpr int LPW = ASTAGE / 1024 / NWAVES;  // loads per wave per operand per stage (4)
+    constexpr int LPA = ASTAGE / 1024 / NWAVES;  // loads per wave per stage: A (4; BM 128: 2)
+    constexpr int LPB = BSTAGE / 1024 / NWAVES;  // ... and B (4)
     constexpr int RPI = 1024 / BK;               // stage rows one instruction fills
     constexpr int CPR = BK / 16;                 // 16-byte chunks per stage row
     constexpr int EPI_LD = WTN + 4;              // staged-epilogue row stride (words)
-    constexpr int SMEM = B_BASE + NSB * BSTAGE;  // 160 KiB, all of the CU's LDS
+    constexpr int SMEM = B_BASE + NSB * BSTAGE;  // 160 KiB, all of the CU's LDS (BM 128: 112)
     constexpr int EPI_BYTES = NWAVES * 16 * EPI_LD * 4;
     static_assert(SMEM <= 160 * 1024, "LDS");
     using M = Mma16x<T>;
     using acc_t = typename M::acc_t;
     using val_t = typename M::scalar_t;
-    constexpr int QCH = (E == EpiKind::Q8) ? BM : 1;
+    constexpr int QCH = (E == EpiKind::Q8) ? BN : 1;  // (BN >= BM)
     static_assert(EPI_BYTES + QCH * 8 <= SMEM, "epilogue staging and channel table do not fit");
     __shared__ __attribute__((aligned(1024))) uint8_t smem[SMEM];
 
@@ -109,18 +115,20 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
     const uint32_t a_num = (uint32_t)(((args.M - m0 < BM ? args.M - m0 : BM) - 1) * lda_b + kb16);
     const uint32_t b_num = (uint32_t)(((args.N - n0 < BN ? args.N - n0 : BN) - 1) * ldb_b + kb16);
 
-    // Loads: wave w fills rows [w*LPW*RPI, +LPW*RPI) of an A stage and of a B
-    // stage; instruction i's rows lie RPI*i below instruction 0's and its
-    // chunk repeats every two instructions (the swizzle).
+    // Loads: wave w fills rows [w*LPA*RPI, +LPA*RPI) of an A stage and likewise
+    // of a B stage; instruction i's rows lie RPI*i below instruction 0's and its
+    // chunk repeats every two instructions (the swizzle; LPA and LPB are even,
+    // so A's and B's chunks agree).
+    static_assert(LPA % 2 == 0 && LPB % 2 == 0, "chunk pattern");
     uint32_t voa[2], vob[2];
     int kch[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int row = (wave * LPW + i) * RPI + lane / CPR;
-        const int ch = (lane % CPR) ^ swz_of<BK>(row);
+        const int ra = (wave * LPA + i) * RPI + lane / CPR, rb = (wave * LPB + i) * RPI + lane / CPR;
+        const int ch = (lane % CPR) ^ swz_of<BK>(ra);
         kch[i] = ch * 16;
-        voa[i] = (uint32_t)(row * lda_b + ch * 16);
-        vob[i] = (uint32_t)(row * ldb_b + ch * 16);
+        voa[i] = (uint32_t)(ra * lda_b + ch * 16);
+        vob[i] = (uint32_t)(rb * ldb_b + ch * 16);
     }
     const uint32_t rsa = (uint32_t)(RPI * lda_b), rsb = (uint32_t)(RPI * ldb_b);
     const bool soff_ok = lda_b >= kb16 && ldb_b >= kb16;
@@ -132,8 +140,8 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
                                    : vob[i % 2] + (uint32_t)(i - i % 2) * rsb;
         const uint8_t *pan = X == 0 ? a_pan : b_pan;
         const uint32_t num = X == 0 ? a_num : b_num;
-        uint8_t *dst = smem + (X == 0 ? slot * ASTAGE : B_BASE + slot * BSTAGE) +
-                       (wave * LPW + i) * 1024;
+        uint8_t *dst = smem + (X == 0 ? slot * ASTAGE + (wave * LPA + i) * 1024
+                                      : B_BASE + slot * BSTAGE + (wave * LPB + i) * 1024);
         if constexpr (decltype(whole)::value) {
             dma16s(pan, num, lo, kb, dst);
         } else {
@@ -225,24 +233,25 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
     // (int8 4096^3 main loop 78.5k against 73.9k shader cycles per
     // workgroup; bf16 157.8k against 146.0k).
     using ZL = std::integral_constant<int, 0>;
-    using LW = std::integral_constant<int, LPW>;
+    using LWA = std::integral_constant<int, LPA>;
+    using LWB = std::integral_constant<int, LPB>;
     auto noload = [](int) {};
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) load1(std::false_type{}, 0, 0, 0, i);
+    for (int i = 0; i < LPA; ++i) load1(std::false_type{}, 0, 0, 0, i);
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) load1(std::false_type{}, 1, 0, 0, i);
+    for (int i = 0; i < LPB; ++i) load1(std::false_type{}, 1, 0, 0, i);
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) load1(std::false_type{}, 0, 1, 1, i);
+    for (int i = 0; i < LPA; ++i) load1(std::false_type{}, 0, 1, 1, i);
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) load1(std::false_type{}, 1, 1, 1, i);
-    wait_vmcnt<2 * LPW>();  // stage 0 landed
+    for (int i = 0; i < LPB; ++i) load1(std::false_type{}, 1, 1, 1, i);
+    wait_vmcnt<LPA + LPB>();  // stage 0 landed
     stage_barrier();
     {
         using NA = std::integral_constant<int, TM>;
         ops(smem, smem + B_BASE, 0, 0, 0, NA{}, std::true_type{}, ZL{}, noload);
     }
 
-    constexpr int NM = (TM / 2) * TN;  // MFMAs per phase (16)
+    constexpr int NM = (TM / 2) * TN;  // MFMAs per phase (16; BM 128: 8)
     constexpr int SPAN = NM * 7 / 8;
     const int ktw = (int)(kbytes / BK);
     // sa: stage kt's A slot (kt % 3).
@@ -257,8 +266,8 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
         // phase 0: sub-step 0, blocks 0-3; read sub-step 1's A 0-3 and B;
         // stage kt+2's A loads
         mfma_rows(0, 0);
-        ops(s_a, s_b, 1, 1, 0, H{}, std::true_type{}, LW{}, ld_a);
-        sched_ops<NM, TM / 2 + TN, LPW, SPAN>();
+        ops(s_a, s_b, 1, 1, 0, H{}, std::true_type{}, LWA{}, ld_a);
+        sched_ops<NM, TM / 2 + TN, LPA, SPAN>();
         // phase 1: sub-step 0, blocks 4-7; read sub-step 1's A 4-7
         mfma_rows(0, TM / 2);
         ops(s_a, s_b, 1, 1, TM / 2, H{}, std::false_type{}, ZL{}, noload);
@@ -272,7 +281,7 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
         for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(af[0][i]));
 #pragma unroll
         for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(bf[0][j]));
-        wait_vmcnt<LPW>();
+        wait_vmcnt<LPA>();
         stage_barrier();
 #pragma unroll
         for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(af[1][i]));
@@ -281,8 +290,8 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
         // phase 3: sub-step 1, blocks 4-7; read stage kt+1's sub-step 0;
         // stage kt+2's B loads
         mfma_rows(1, TM / 2);
-        ops(n_a, n_b, 0, 0, 0, FA{}, std::true_type{}, LW{}, ld_b);
-        sched_ops<NM, TM + TN, LPW, SPAN>();
+        ops(n_a, n_b, 0, 0, 0, FA{}, std::true_type{}, LWB{}, ld_b);
+        sched_ops<NM, TM + TN, LPB, SPAN>();
     };
     // Stages whose loads (of stage kt+2) lie wholly inside K take the
     // scalar-offset loads.
@@ -350,13 +359,14 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
     // (requant_pack4's fast tier needs no overflow check then).
     bool tame = true;
     if constexpr (E == EpiKind::Q8) {
-        static_assert(WTN == 64 && WTM == 128, "one channel per lane (columns) or two (rows)");
+        static_assert(WTN == 64 && (WTM == 64 || WTM == 128),
+                      "one channel per lane (columns), one or two (rows)");
         bool bad;
         if (ep.axis) {
             bad = !(__builtin_fabsf(q_scale[wn * WTN + lane]) < 0x1p100f);
         } else {
             bad = !(__builtin_fabsf(q_scale[wm * WTM + lane]) < 0x1p100f) ||
-                  !(__builtin_fabsf(q_scale[wm * WTM + 64 + lane]) < 0x1p100f);
+                  (WTM == 128 && !(__builtin_fabsf(q_scale[wm * WTM + 64 + lane]) < 0x1p100f));
         }
         tame = __builtin_amdgcn_ballot_w64(bad) == 0;
     }
@@ -464,27 +474,36 @@ void mma16_kernel(const MmaArgs args, const EpiParams ep) {
     }
 }
 
-template <InType T, EpiKind E>
+template <InType T, EpiKind E, int BM>
 static hipError_t launch16(const MmaArgs &args, const EpiParams &ep, hipStream_t stream) {
     if ((args.pn != 0 && args.pn != 256) || args.splits > 1) return hipErrorInvalidValue;
     const int esz = T == InType::I8 ? 1 : 2;
-    if (!panels_fit(256, 256, args.lda * esz, args.ldb * esz, (int64_t)args.K * esz))
+    if (!panels_fit(BM, 256, args.lda * esz, args.ldb * esz, (int64_t)args.K * esz))
         return hipErrorInvalidValue;
-    const int tiles = ((args.M + 255) / 256) * ((args.N + 255) / 256);
-    hipLaunchKernelGGL((mma16_kernel<T, E>), dim3(tiles, 1, args.batch), dim3(512), 0, stream,
+    const int tiles = ((args.M + BM - 1) / BM) * ((args.N + 255) / 256);
+    hipLaunchKernelGGL((mma16_kernel<T, E, BM>), dim3(tiles, 1, args.batch), dim3(512), 0, stream,
                        args, ep);
     return hipGetLastError();
 }
 
-hipError_t launch_mma16(InType in, const MmaArgs &args, const EpiParams &ep, hipStream_t stream) {
+template <int BM>
+static hipError_t launch16_bm(InType in, const MmaArgs &args, const EpiParams &ep,
+                              hipStream_t stream) {
     if (in == InType::I8) {
-        if (ep.kind == EpiKind::I32) return launch16<InType::I8, EpiKind::I32>(args, ep, stream);
-        if (ep.kind == EpiKind::Q8) return launch16<InType::I8, EpiKind::Q8>(args, ep, stream);
+        if (ep.kind == EpiKind::I32) return launch16<InType::I8, EpiKind::I32, BM>(args, ep, stream);
+        if (ep.kind == EpiKind::Q8) return launch16<InType::I8, EpiKind::Q8, BM>(args, ep, stream);
     } else if (in == InType::BF16) {
-        if (ep.kind == EpiKind::F32) return launch16<InType::BF16, EpiKind::F32>(args, ep, stream);
-        if (ep.kind == EpiKind::BF16) return launch16<InType::BF16, EpiKind::BF16>(args, ep, stream);
+        if (ep.kind == EpiKind::F32) return launch16<InType::BF16, EpiKind::F32, BM>(args, ep, stream);
+        if (ep.kind == EpiKind::BF16)
+            return launch16<InType::BF16, EpiKind::BF16, BM>(args, ep, stream);
     }
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_mma16(InType in, Tile tile, const MmaArgs &args, const EpiParams &ep,
+                        hipStream_t stream) {
+    return tile == Tile::T128x256w8m16 ? launch16_bm<128>(in, args, ep, stream)
+                                       : launch16_bm<256>(in, args, ep, stream);
 }
 
 }  // namespace gk

@@ -984,6 +984,7 @@ static hipError_t launch_tile(Tile tile, const MmaArgs &args, const EpiParams &e
     case Tile::T256x352w8k128: return launch_one<T, E, 256, 352, 2, 4, 2, false, 128>(args, ep, stream);
     case Tile::T256x256w8m16: break;  // mma16.hip (launch_mma dispatches it first)
     case Tile::T256x352w8m16: break;  // mma16w.hip (likewise)
+    case Tile::T128x256w8m16: break;  // mma16.hip
     }
     return hipErrorInvalidValue;
 }
