@@ -1062,9 +1062,14 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     const bool gemv_cols = vector_route && !skinny_ok && short_side <= kGemvColsMaxVec &&
                            mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
                            std::max(M, N) * (int64_t)esz >= 16;
-    const bool cols_pack_vec = gemv_cols && (vec_is_a ? A : Bt).ks != 1;
-    const bool pack_a = gemv_cols ? vec_is_a && cols_pack_vec : !a_ok && !(skinny_ok && vec_is_a);
-    const bool pack_b = gemv_cols ? !vec_is_a && cols_pack_vec : !b_ok && !(skinny_ok && !vec_is_a);
+    // The skinny kernel likewise, with its sums added in a second launch (bf16
+    // 8 x 4096 x 4096: 10.6 us against 25.1; 16 x 1024 x 1024: 5.3 against 8.8).
+    const bool skinny_cols = skinny_ok && mat_op.rs == 1 && mat_op.ks != 1 &&
+                             kbytes >= kGemvColsMinBytes && std::max(M, N) >= kSkinnyColsMinRows;
+    const bool cols = gemv_cols || skinny_cols;
+    const bool cols_pack_vec = cols && (vec_is_a ? A : Bt).ks != 1;
+    const bool pack_a = cols ? vec_is_a && cols_pack_vec : !a_ok && !(skinny_ok && vec_is_a);
+    const bool pack_b = cols ? !vec_is_a && cols_pack_vec : !b_ok && !(skinny_ok && !vec_is_a);
     // Split K.  Float products split by the element shape only (a batched
     // element sums in the same order as the standalone product); i8 sums do
     // not depend on the split (wrapping addition), so an i8 batch that fills
@@ -1133,6 +1138,8 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         splits > 1 ? (size_t)round_up64(zchunk * elem_part, 256)
         : gemv_cols
             ? (size_t)gemv_cols_part_bytes(in, std::max(M, N), k, (int)short_side, batch, g_num_cus)
+        : skinny_cols
+            ? (size_t)skinny_cols_part_bytes(in, std::max(M, N), k, (int)short_side, batch, g_num_cus)
             : 0;
 
     uint8_t *part = nullptr;
@@ -1174,7 +1181,8 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         g.K = (int32_t)k;
         g.cus = g_num_cus;
         g.batch = (int32_t)batch;
-        e = skinny_ok   ? launch_skinny(in, g, eg, tl_stream)
+        e = skinny_cols ? launch_skinny_cols(in, g, eg, tl_stream)
+            : skinny_ok ? launch_skinny(in, g, eg, tl_stream)
             : gemv_cols ? launch_gemv_cols(in, g, eg, tl_stream)
                         : launch_gemv(in, g, eg, tl_stream);
         if (e != hipSuccess) return hip_fail(e, skinny_ok ? "skinny launch" : "gemv launch");

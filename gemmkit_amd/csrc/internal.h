@@ -136,8 +136,8 @@ struct GemvArgs {
     int32_t cus;           // compute units of the device (persistent grid size)
     int32_t batch;         // batch elements (grid y), at most kMaxGridZ
     int64_t bsm, bsv;      // batch strides of mat and vec in elements
-    int64_t mks;           // k stride of mat: 1, or any with ld == 1 (launch_gemv_cols only)
-    void *part;            // gemv_cols_part_bytes() of scratch, or nullptr (launch_gemv_cols only)
+    int64_t mks;           // k stride of mat: 1, or any with ld == 1 (launch_gemv_cols, launch_skinny_cols)
+    void *part;            // their *_part_bytes() of scratch, or nullptr
     // Output element (vector j, matrix row r) of batch element z is stored as
     // the epilogue's (row j, column r) of element z: at c + z*bsc + j*rsc +
     // r*csc of the EpiParams.  Each element's arithmetic does not depend on
@@ -183,6 +183,14 @@ hipError_t launch_gemv_cols(InType in, const GemvArgs &g, const EpiParams &ep, h
 constexpr int64_t kSkinnyLdsMax = 128 * 1024;
 int64_t skinny_lds_bytes(InType in, int64_t K, int nvec);
 hipError_t launch_skinny(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
+
+// The same products over a matrix of unit row stride (ld == 1, k stride mks) with
+// at least kSkinnyColsMinRows rows and k-contiguous vectors, both with any
+// alignment, bit for bit; g.part must hold skinny_cols_part_bytes().
+constexpr int kSkinnyColsMinRows = 8;
+int64_t skinny_cols_part_bytes(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus);
+hipError_t launch_skinny_cols(InType in, const GemvArgs &g, const EpiParams &ep,
+                              hipStream_t stream);
 
 // Pack `batch` (at most kMaxGridZ) strided rows x K operands, element (r, p) of
 // element z at src + z*bs + r*rs + p*cs, into a k-contiguous buffer with row

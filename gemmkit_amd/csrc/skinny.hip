@@ -397,6 +397,263 @@ static hipError_t skinny_go(const GemvArgs &g, const EpiParams &ep, hipStream_t 
     return hipGetLastError();
 }
 
+// ---- skinny_cols ------------------------------------------------------------
+// The same products with a matrix of unit row stride (element (r, p) at
+// r + p*mks, any mks and alignment; x * W with W row-major) and k-contiguous
+// vectors (any alignment), read in place.
+//
+// A lane loads 8 bytes, RPL rows, at one k (16 lanes side by side a run of 128
+// bytes), for each k of its 16-byte chunk; byte permutes in registers turn them
+// into RPL matrix-core operands, operand t holding rows RPL*i + t of the lanes
+// i.  The kernel above sums a row in eight parts: four K ranges, each the sum
+// of the even 16-byte chunks of its 128-byte steps (MFMA h = 0) and of the odd
+// ones (h = 1).  Here every part is a wave of its own -- workgroup = (part, 16*RPL
+// rows) -- which stores its sums, and cols_sum adds the parts in the order above:
+// results equal that kernel's on a packed copy bit for bit.  i8, whose sums have no
+// order, takes more ranges when the parts are few for the CUs.
+//
+// Bound by streaming the matrix once, against three passes when it is packed first
+// (copies in turn, together beyond the caches; second launch included): bf16
+// 8 x 4096 x 4096 10.6 us against 25.1, 4 x 4096 x 11008 18.4 (4.9 TB/s) against
+// 51, 16 x 1024 x 1024 5.3 against 8.8; f32 4 x 4096 x 11008 36.1 (5.0 TB/s) against
+// 122, 8 x 1024 x 16384 19.4 against 45; i8 8 x 11008 x 4096 13.0 against 36.5.
+typedef int v2i_s __attribute__((ext_vector_type(2)));
+typedef int v2i_sany __attribute__((ext_vector_type(2), aligned(1)));
+typedef int v4i_sany __attribute__((ext_vector_type(4), aligned(1)));
+
+template <InType T>
+struct SkCols;
+
+template <>
+struct SkCols<InType::F32> {
+    static constexpr int PF = 8;  // k steps per batch of loads (64 registers)
+    using acc_t = v4f_s;
+    using elem_t = uint32_t;
+    // m[e]: the lane's RPL rows at k = e of its chunk; x: the chunk of its vector.
+    __device__ __forceinline__ static void step(const v2i_s (&m)[4], v4i_s x, acc_t (&acc)[2]) {
+        const v4f_s xf = __builtin_bit_cast(v4f_s, x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__int_as_float(m[e][t]), xf[e],
+                                                              acc[t], 0, 0, 0);
+    }
+};
+
+template <>
+struct SkCols<InType::BF16> {
+    static constexpr int PF = 4;
+    using acc_t = v4f_s;
+    using elem_t = uint16_t;
+    __device__ __forceinline__ static void step(const v2i_s (&m)[8], v4i_s x, acc_t (&acc)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            v4i_s w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                w[i] = (int)__builtin_amdgcn_perm((uint32_t)m[2 * i + 1][t / 2],
+                                                  (uint32_t)m[2 * i][t / 2],
+                                                  t % 2 ? 0x07060302u : 0x05040100u);
+            acc[t] = Mma16<InType::BF16>::step(w, x, acc[t]);
+        }
+    }
+};
+
+template <>
+struct SkCols<InType::I8> {
+    static constexpr int PF = 2;
+    using acc_t = v4i_s;
+    using elem_t = uint8_t;
+    __device__ __forceinline__ static void step(const v2i_s (&m)[16], v4i_s x, acc_t (&acc)[8]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            v4i_s w[4];  // 4 x 4 byte transposes: four k of a row side by side
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const uint32_t i0 = m[4 * p][c], i1 = m[4 * p + 1][c];
+                const uint32_t i2 = m[4 * p + 2][c], i3 = m[4 * p + 3][c];
+                const uint32_t t0 = __builtin_amdgcn_perm(i1, i0, 0x05010400u);
+                const uint32_t t1 = __builtin_amdgcn_perm(i1, i0, 0x07030602u);
+                const uint32_t u0 = __builtin_amdgcn_perm(i3, i2, 0x05010400u);
+                const uint32_t u1 = __builtin_amdgcn_perm(i3, i2, 0x07030602u);
+                w[0][p] = (int)__builtin_amdgcn_perm(u0, t0, 0x05040100u);
+                w[1][p] = (int)__builtin_amdgcn_perm(u0, t0, 0x07060302u);
+                w[2][p] = (int)__builtin_amdgcn_perm(u1, t1, 0x05040100u);
+                w[3][p] = (int)__builtin_amdgcn_perm(u1, t1, 0x07060302u);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc[4 * c + t] = Mma16<InType::I8>::step(w[t], x, acc[4 * c + t]);
+        }
+    }
+};
+
+template <InType T>
+__global__ __launch_bounds__(64) void skinny_cols(const GemvArgs g, int ranges) {
+    using Sc = SkCols<T>;
+    using elem_t = typename Sc::elem_t;
+    using val_t = typename Mma16<T>::val_t;
+    constexpr int EPC = 16 / (int)sizeof(elem_t), RPL = 8 / (int)sizeof(elem_t);
+    constexpr int ROWS = 16 * RPL, STEPK = kSkStep / (int)sizeof(elem_t), PF = Sc::PF;
+    const int lane = threadIdx.x, li = lane & 15, lg = lane >> 4;
+    const unsigned groups = (unsigned)(((int64_t)g.R + ROWS - 1) / ROWS);
+    const int unit = (int)(blockIdx.x / groups), h = unit & 1, range = unit >> 1;
+    const int64_t rg = (int64_t)(blockIdx.x % groups) * ROWS, zb = blockIdx.y;
+    // Rows start RPL before R at the latest, so every load stays inside the
+    // matrix (the caller ensures R >= RPL); overlapping lanes form, and store,
+    // the same sums.
+    const auto row_of = [&](int i) {
+        return rg + RPL * i + RPL <= g.R ? rg + RPL * i : (int64_t)g.R - RPL;
+    };
+    const int nk = (int)(((int64_t)g.K + STEPK - 1) / STEPK);
+    const int kseg = (nk + ranges - 1) / ranges;
+    const int ks0 = range * kseg, ks1 = ks0 + kseg < nk ? ks0 + kseg : nk;
+    const int whole = g.K / STEPK, kfull = ks1 < whole ? ks1 : whole;  // whole steps: [ks0, kfull)
+    const int64_t k0 = (2 * lg + h) * EPC;  // this lane's chunk of a step
+    const elem_t *mat = (const elem_t *)g.mat + zb * g.bsm + row_of(li) + k0 * g.mks;
+    // (columns past nvec repeat the last vector; they are not stored)
+    const elem_t *vec = (const elem_t *)g.vec + zb * g.bsv +
+                        (int64_t)(li < g.nvec ? li : g.nvec - 1) * g.vld + k0;
+
+    typename Sc::acc_t acc[RPL] = {};
+    // Two batches in turn, the next one's loads in flight while one is
+    // multiplied.  All loads of a batch are issued before any is used; steps past
+    // the end load the last one again and are left out.
+    auto load = [&](int s, v2i_s (&m)[PF][EPC], v4i_s (&x)[PF]) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            const int64_t k = (int64_t)(s + u < kfull ? s + u : kfull - 1) * STEPK;
+            x[u] = *(const v4i_sany *)(vec + k);
+#pragma unroll
+            for (int e = 0; e < EPC; ++e) m[u][e] = *(const v2i_sany *)(mat + (k + e) * g.mks);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mul = [&](int s, const v2i_s (&m)[PF][EPC], const v4i_s (&x)[PF]) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u)
+            if (s + u < kfull) Sc::step(m[u], x[u], acc);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (ks0 < kfull) {
+        v2i_s m0[PF][EPC], m1[PF][EPC];
+        v4i_s x0[PF], x1[PF];
+        load(ks0, m0, x0);
+        for (int s = ks0; s < kfull; s += 2 * PF) {
+            if (s + PF < kfull) load(s + PF, m1, x1);
+            mul(s, m0, x0);
+            if (s + PF >= kfull) break;
+            if (s + 2 * PF < kfull) load(s + 2 * PF, m0, x0);
+            mul(s + PF, m1, x1);
+        }
+    }
+    if (whole >= ks0 && whole < ks1) {  // the last step, zeros past K
+        v2i_s m[EPC];
+        elem_t v[EPC];
+        const int64_t k = (int64_t)whole * STEPK;
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) {
+            const bool in = k + k0 + e < g.K;
+            m[e] = v2i_s{0, 0};
+            v[e] = elem_t(0);
+            if (in) {
+                m[e] = *(const v2i_sany *)(mat + (k + e) * g.mks);
+                v[e] = vec[k + e];
+            }
+        }
+        v4i_s x;
+        __builtin_memcpy(&x, v, 16);
+        Sc::step(m, x, acc);
+    }
+    if (li < g.nvec) {
+        val_t *out = (val_t *)g.part + ((zb * 2 * ranges + unit) * g.nvec + li) * g.R;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            val_t v[RPL];
+#pragma unroll
+            for (int t = 0; t < RPL; ++t) v[t] = acc[t][q];
+            __builtin_memcpy(out + row_of(4 * lg + q), v, sizeof(v));
+        }
+    }
+}
+
+// Adds the parts [element][range][h][vector][row], one output per thread.
+template <InType T, EpiKind E, int RANGES>
+__global__ __launch_bounds__(64) void cols_sum(const GemvArgs g, const EpiParams ep) {
+    using val_t = typename Mma16<T>::val_t;
+    const int64_t r = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    const int j = blockIdx.y;
+    const int64_t zb = blockIdx.z;
+    if (r >= g.R) return;
+    val_t v[2 * RANGES];
+#pragma unroll
+    for (int u = 0; u < 2 * RANGES; ++u)
+        v[u] = ((const val_t *)g.part)[((zb * 2 * RANGES + u) * g.nvec + j) * g.R + r];
+    val_t sum = v[0] + v[1];
+#pragma unroll
+    for (int u = 1; u < RANGES; ++u) sum += v[2 * u] + v[2 * u + 1];
+    Store<E>::apply(ep, zb, j, (int)r, sum);
+}
+
+// K ranges: 4 for floats (the row kernel's order); i8 up to 16 while that leaves
+// fewer than four waves per CU, a batch of loads to each and a scratch no larger
+// than a quarter of the matrix.
+static int skinny_cols_ranges(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus) {
+    int ranges = 4;
+    if (in != InType::I8) return ranges;
+    const int64_t groups = (R + 127) / 128 * batch;
+    while (ranges < 16 && groups * 2 * ranges < 4 * (int64_t)(cus > 0 ? cus : 256) &&
+           K >= (int64_t)2 * ranges * 128 * SkCols<InType::I8>::PF &&
+           4 * ranges * nvec * 4 * 4 <= K)
+        ranges *= 2;
+    return ranges;
+}
+
+int64_t skinny_cols_part_bytes(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus) {
+    return 2 * skinny_cols_ranges(in, R, K, nvec, batch, cus) * batch * nvec * R * 4;
+}
+
+template <InType T, EpiKind E>
+static hipError_t skinny_cols_go(const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {
+    constexpr int ROWS = 16 * 8 / (T == InType::I8 ? 1 : (T == InType::BF16 ? 2 : 4));
+    const int ranges = skinny_cols_ranges(T, g.R, g.K, g.nvec, g.batch, g.cus);
+    const int64_t groups = ((int64_t)g.R + ROWS - 1) / ROWS;
+    hipLaunchKernelGGL((skinny_cols<T>), dim3((unsigned)(groups * 2 * ranges), (unsigned)g.batch),
+                       dim3(64), 0, stream, g, ranges);
+    const dim3 grid((unsigned)(((int64_t)g.R + 63) / 64), (unsigned)g.nvec, (unsigned)g.batch);
+    if constexpr (T == InType::I8) {
+        if (ranges == 16)
+            hipLaunchKernelGGL((cols_sum<T, E, 16>), grid, dim3(64), 0, stream, g, ep);
+        else if (ranges == 8)
+            hipLaunchKernelGGL((cols_sum<T, E, 8>), grid, dim3(64), 0, stream, g, ep);
+    }
+    if (ranges == 4) hipLaunchKernelGGL((cols_sum<T, E, 4>), grid, dim3(64), 0, stream, g, ep);
+    return hipGetLastError();
+}
+
+hipError_t launch_skinny_cols(InType in, const GemvArgs &g, const EpiParams &ep,
+                              hipStream_t stream) {
+    if (g.nvec < 1 || g.nvec > 16 || g.R < kSkinnyColsMinRows || g.ld != 1 || g.vks != 1 ||
+        !g.part || g.batch < 1 || g.batch > kMaxGridZ)
+        return hipErrorInvalidValue;
+    switch (in) {
+    case InType::I8:
+        if (ep.kind == EpiKind::I32) return skinny_cols_go<InType::I8, EpiKind::I32>(g, ep, stream);
+        if (ep.kind == EpiKind::Q8) return skinny_cols_go<InType::I8, EpiKind::Q8>(g, ep, stream);
+        break;
+    case InType::F32:
+        if (ep.kind == EpiKind::F32) return skinny_cols_go<InType::F32, EpiKind::F32>(g, ep, stream);
+        break;
+    case InType::BF16:
+        if (ep.kind == EpiKind::F32) return skinny_cols_go<InType::BF16, EpiKind::F32>(g, ep, stream);
+        if (ep.kind == EpiKind::BF16)
+            return skinny_cols_go<InType::BF16, EpiKind::BF16>(g, ep, stream);
+        break;
+    }
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_skinny(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {
     // The matrix rows are addressed as unsigned 32-bit offsets from an item's
     // first row, so its row stride must be non-negative (the vectors may

@@ -1,0 +1,92 @@
+"""Skinny products over a matrix of unit row stride (a few rows times W with W
+row-major): equal bit for bit to the same call with W k-contiguous, so in the
+same summing order, on ragged columns and K, unaligned rows, empty K ranges,
+strided vectors, either side as the vectors, batches and every epilogue."""
+import pytest
+import torch
+
+import gemmkit_amd as gk
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f32": torch.float32, "bf16": torch.bfloat16, "i8": torch.int8}
+
+
+def values(n, dt, seed, dev):
+    g = torch.Generator().manual_seed(seed)
+    if dt == torch.int8:
+        return torch.randint(-128, 128, (n,), generator=g, dtype=dt).to(dev)
+    return torch.randn(n, generator=g).to(dt).to(dev)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "i8"])
+# (vectors, k, n): fewer rows than a lane group, one and many groups, K below a
+# step per range, ending inside a chunk, on a step, on a batch of loads, and
+# (i8) long enough for 8 and 16 ranges
+@pytest.mark.parametrize("shape", [(2, 1024, 17), (3, 1025, 33), (5, 1100, 64), (8, 2048, 1000),
+                                   (9, 1536, 129), (16, 1984, 40), (4, 8200, 75), (2, 6144, 300),
+                                   (15, 1601, 2050), (2, 16384, 65), (4, 4095, 257)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_unit_row_stride_equals_k_contiguous(dev, dtype, shape):
+    m, k, n = shape
+    dt = DT[dtype]
+    pad = 16 // dt.itemsize
+    kp = (k + pad - 1) // pad * pad
+    a, w = values(m * k, dt, 1, dev), values(k * n, dt, 2, dev).view(k, n)
+    a0 = torch.zeros(m, kp, dtype=dt, device=dev)
+    a0[:, :k] = a.view(m, k)
+    w0 = torch.zeros(n, kp, dtype=dt, device=dev)
+    w0[:, :k] = w.T
+    off = 1 + torch.zeros(1 + k * (n + 3), dtype=dt, device=dev)  # odd base, padded rows
+    off[1:].view(k, n + 3)[:, :n] = w
+    at = a.view(m, k).T.contiguous()  # vectors side by side
+    cdt = torch.int32 if dt == torch.int8 else dt
+    f = gk.gemm_i8_unchecked if dt == torch.int8 else gk.gemm_unchecked
+    for alpha, beta in ((1, 0), (3, 2)):
+        c0 = torch.arange(m * n, device=dev).remainder(7).to(cdt)
+        outs = []
+        for x, rsa, csa, b, rsb, csb, bo in ((a0, kp, 1, w0, 1, kp, 0), (a, k, 1, w, n, 1, 0),
+                                             (a, k, 1, off, n + 3, 1, 1), (at, 1, m, w, n, 1, 0)):
+            c = c0.clone()
+            f(m, k, n, alpha, x, rsa, csa, b, rsb, csb, beta, c, n, 1, b_off=bo)
+            outs.append(c)
+        # the transposed product: W^T (n x k, column-major) times the vectors
+        c = c0.view(m, n).T.contiguous().reshape(-1)
+        f(n, k, m, alpha, w, 1, n, a, 1, k, beta, c, m, 1)
+        outs.append(c.view(n, m).T.contiguous().reshape(-1))
+        for c in outs[1:]:
+            assert torch.equal(c.view(torch.uint8), outs[0].view(torch.uint8))
+    if dt == torch.int8:
+        want = a.view(m, k).double() @ w.double()
+        assert torch.equal((outs[0] - 2 * c0).double(), 3 * want.reshape(-1))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_batch_and_packed_equal_standalone(dev, dtype):
+    dt, batch, m, k, n = DT[dtype], 5, 6, 2052, 75
+    a, b = values(batch * m * k, dt, 3, dev), values(batch * k * n, dt, 4, dev)
+    c = torch.zeros(batch * m * n, dtype=dt, device=dev)
+    gk.gemm_batched_unchecked(batch, m, k, n, 1.0, a, k, 1, m * k, b, n, 1, k * n, 0.0, c, n, 1,
+                              m * n)
+    for z in range(batch):
+        one, pk = (torch.zeros(m * n, dtype=dt, device=dev) for _ in range(2))
+        gk.gemm_unchecked(m, k, n, 1.0, a, k, 1, b, n, 1, 0.0, one, n, 1, a_off=z * m * k,
+                          b_off=z * k * n)
+        assert torch.equal(c[z * m * n:(z + 1) * m * n], one)
+        w = gk.prepack_rhs(gk.MatRef.from_row_major(b[z * k * n:(z + 1) * k * n], k, n))
+        gk.gemm_packed_b(1.0, gk.MatRef.from_row_major(a[z * m * k:(z + 1) * m * k], m, k), w, 0.0,
+                         gk.MatMut.from_col_major(pk, m, n))
+        assert torch.equal(pk.view(n, m).T.reshape(-1), one)
+
+
+def test_nonfinite_columns_stay_apart(dev):
+    """A row of infinities or NaN reaches its own outputs only, past K neither."""
+    m, k, n = 3, 1030, 50
+    a, w = values(m * k, torch.bfloat16, 5, dev), values(k * n, torch.bfloat16, 6, dev)
+    w = torch.cat([w, torch.full((64 * n,), float("nan"), dtype=w.dtype, device=dev)])
+    w.view(-1, n)[:k, 7] = float("inf")
+    w.view(-1, n)[:k, 49] = float("nan")
+    c = torch.zeros(m, n, dtype=torch.bfloat16, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, a, k, 1, w, n, 1, 0.0, c, n, 1)
+    bad = ~torch.isfinite(c)
+    assert bad[:, [7, 49]].all() and bad.sum() == 2 * m
