@@ -874,6 +874,8 @@ constexpr int64_t kF32xMinK = 128;
 // Shortest row the unit-row-stride GEMV takes: one 16-byte chunk for each of
 // a workgroup's 64 slots.
 constexpr int64_t kGemvColsMinBytes = 1024;
+// ... and most rows (a grid of at most 2^32 threads).
+constexpr int64_t kColsMaxRows = 1 << 26;
 
 int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int64_t n,
             const void *a, int64_t rsa, int64_t csa, int64_t bsa, const void *b, int64_t rsb,
@@ -1049,27 +1051,59 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // when they are not k-contiguous.
     const bool vec_is_a = M <= N;
     const bool gemv_first = gemv_beats_skinny(in, short_side, kbytes);
+    // Vectors beyond the LDS of a workgroup: 5..8 (bf16 3..8) on skinny_long, fewer on
+    // the GEMV (f32 4 x 16384 x 600: 20 us against 26; bf16 14.3 against 13.0); more of them, whose L2 reads are as large as the matrix's
+    // in 16-row items and twice that in 8-row ones, where 16-row items fill the CUs
+    // and, for bf16, rows are at most 16 KiB: 16 x 4096 x 4096 10.0 us against 12.7
+    // on the split matrix-core tiles, f32 18.1 against 42, i8 16 x 11008 x 4096 13.4
+    // against 14.3; bf16 16 x 11008 x 4096 22.9 against 20.4 and f32 16 x 16384 x
+    // 2500 75 against 51 stay there.  i8, whose sums have no order, takes it with
+    // 5..8 vectors already where the LDS would hold one workgroup a CU (8 x 11008
+    // x 4096: 11.5 against 18.9), and reads a row-major matrix in place in any case.
+    const Opnd &mat_op = vec_is_a ? Bt : A;
+    const int64_t long_side = std::max(M, N);
+    const bool mat_cols = mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
+                          long_side <= kColsMaxRows;
+    const bool long_vec = skinny_is_long(in, k, (int)std::min<int64_t>(short_side, 16));
+    const bool long_ok =
+        short_side <= 8 ? short_side > (in == InType::BF16 ? 2 : kGemvColsMaxVec)
+                        : (in == InType::I8 && mat_cols) ||
+                              (long_side >= 16 * (int64_t)(g_num_cus > 0 ? g_num_cus : 256) &&
+                               (in != InType::BF16 || kbytes <= 16384));
     const bool skinny_ok = short_side >= 2 && short_side <= 16 && !gemv_first &&
-                           skinny_enabled() && k_fits &&
-                           skinny_lds_bytes(in, k, (int)short_side) <= kSkinnyLdsMax;
+                           skinny_enabled() && k_fits && (!long_vec || long_ok);
+    const bool skinny_long =
+        skinny_ok &&
+        (long_vec || (in == InType::I8 && short_side > kGemvColsMaxVec && short_side <= 8 &&
+                      (vec_is_a ? a_ok : b_ok) &&
+                      skinny_lds_bytes(in, k, (int)short_side) > 80 * 1024));
     const bool vector_route = skinny_ok || short_side <= 8;
     // A GEMV whose matrix has unit row stride (x * W with W row-major) reads
     // both operands in place instead of packing the matrix first, three
     // passes over it (bf16 1 x 4096 x 11008: 17 against 55 us), once K is long
     // enough for every slot of its workgroups to have a chunk (below that most
     // of its lanes would idle); same bits either way.
-    const Opnd &mat_op = vec_is_a ? Bt : A;
-    const bool gemv_cols = vector_route && !skinny_ok && short_side <= kGemvColsMaxVec &&
-                           mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
-                           std::max(M, N) * (int64_t)esz >= 16;
+    // Its slots walk K in series, about 0.85 us per batch of loads: a narrow matrix of
+    // long K is packed as before (bf16 2 x 40000 x 300: 36 us against 50; f32
+    // 4 x 16384 x 100: 25 against 28, x 600: 35 against 26).
     // The skinny kernel likewise, with its sums added in a second launch (bf16
-    // 8 x 4096 x 4096: 10.6 us against 25.1; 16 x 1024 x 1024: 5.3 against 8.8).
-    const bool skinny_cols = skinny_ok && mat_op.rs == 1 && mat_op.ks != 1 &&
-                             kbytes >= kGemvColsMinBytes && std::max(M, N) >= kSkinnyColsMinRows;
+    // 8 x 4096 x 4096: 10.6 us against 25.1; 16 x 1024 x 1024: 5.3 against 8.8); i8
+    // sums have no order, so it takes long K from the GEMV there (1 x 16384 x 1024:
+    // two vectors on it 9.9 us, one on the GEMV 16.2).
+    const bool skinny_cols =
+        mat_cols && long_side >= kSkinnyColsMinRows &&
+        (skinny_ok || (in == InType::I8 && short_side <= kGemvColsMaxVec && k > 8192 && k_fits &&
+                       skinny_enabled()));
+    const int64_t rounds = gemv_cols_rounds(in, k, (int)short_side);
+    const bool gemv_cols = vector_route && !skinny_ok && !skinny_cols &&
+                           short_side <= kGemvColsMaxVec && mat_cols &&
+                           long_side * (int64_t)esz >= 16 &&
+                           (rounds <= 16 || long_side * kbytes >= rounds * (3 << 18));
     const bool cols = gemv_cols || skinny_cols;
     const bool cols_pack_vec = cols && (vec_is_a ? A : Bt).ks != 1;
-    const bool pack_a = cols ? vec_is_a && cols_pack_vec : !a_ok && !(skinny_ok && vec_is_a);
-    const bool pack_b = cols ? !vec_is_a && cols_pack_vec : !b_ok && !(skinny_ok && !vec_is_a);
+    const bool vec_in_place = skinny_ok && !skinny_long;  // staged from any strides
+    const bool pack_a = cols ? vec_is_a && cols_pack_vec : !a_ok && !(vec_in_place && vec_is_a);
+    const bool pack_b = cols ? !vec_is_a && cols_pack_vec : !b_ok && !(vec_in_place && !vec_is_a);
     // Split K.  Float products split by the element shape only (a batched
     // element sums in the same order as the standalone product); i8 sums do
     // not depend on the split (wrapping addition), so an i8 batch that fills
@@ -1182,6 +1216,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         g.cus = g_num_cus;
         g.batch = (int32_t)batch;
         e = skinny_cols ? launch_skinny_cols(in, g, eg, tl_stream)
+            : skinny_long ? launch_skinny_long(in, g, eg, tl_stream)
             : skinny_ok ? launch_skinny(in, g, eg, tl_stream)
             : gemv_cols ? launch_gemv_cols(in, g, eg, tl_stream)
                         : launch_gemv(in, g, eg, tl_stream);

@@ -793,6 +793,11 @@ static hipError_t gemv_cols_nv(const GemvArgs &g, const EpiParams &ep, hipStream
     return cols_nv<T, E, 4>(g, ep, stream);
 }
 
+int64_t gemv_cols_rounds(InType in, int64_t K, int nvec) {
+    const int64_t epc = 16 / (int64_t)in_size(in);
+    return K / epc / (64 * (cols_wgrow(in, nvec, K) ? 4 : 1) * cols_unroll(in, nvec));
+}
+
 // K is split over workgroups when a slot has more than one batch of loads and
 // the column groups are few for the CUs: 1 x 4096 x 4096 (64 groups) 10.0 against
 // 12.4 us in one workgroup per group, x 1024 (16 groups) 8.1 against 11.5, i8

@@ -175,6 +175,7 @@ hipError_t launch_gemv(InType in, const GemvArgs &g, const EpiParams &ep, hipStr
 // operands.  Few columns run K split over workgroups through g.part, which
 // must hold gemv_cols_part_bytes() (0: not split).
 constexpr int kGemvColsMaxVec = 4;
+int64_t gemv_cols_rounds(InType in, int64_t K, int nvec);  // batches of loads in series
 int64_t gemv_cols_part_bytes(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus);
 hipError_t launch_gemv_cols(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
 
@@ -183,6 +184,13 @@ hipError_t launch_gemv_cols(InType in, const GemvArgs &g, const EpiParams &ep, h
 constexpr int64_t kSkinnyLdsMax = 128 * 1024;
 int64_t skinny_lds_bytes(InType in, int64_t K, int nvec);
 hipError_t launch_skinny(InType in, const GemvArgs &g, const EpiParams &ep, hipStream_t stream);
+
+// Where the vectors would leave a CU's LDS room for one workgroup of launch_skinny:
+// launch_skinny_long reads them from L2 instead (k-contiguous, 16-byte aligned rows
+// zero-padded to 16 bytes like the matrix's).
+bool skinny_is_long(InType in, int64_t K, int nvec);
+hipError_t launch_skinny_long(InType in, const GemvArgs &g, const EpiParams &ep,
+                              hipStream_t stream);
 
 // The same products over a matrix of unit row stride (ld == 1, k stride mks) with
 // at least kSkinnyColsMinRows rows and k-contiguous vectors, both with any

@@ -397,6 +397,160 @@ static hipError_t skinny_go(const GemvArgs &g, const EpiParams &ep, hipStream_t 
     return hipGetLastError();
 }
 
+// ---- skinny_long ------------------------------------------------------------
+// skinny_mfma's loads and matrix-core layout for vectors that would fill a CU's
+// LDS: each wave reads its vector chunks beside the matrix's, from L2, so nothing
+// is staged and the eight waves of a workgroup, one K range each, are the only
+// limit on the loads in flight.  The vectors are k-contiguous with aligned rows.
+// Every kSkPF steps the accumulators are added to running sums: a sum is then a
+// chain of a few steps inside a chain of K / (8 waves * kSkPF steps): error against
+// 64 bits 1.67e-7 rms at f32 8 x 11008 (standard normal times 1/sqrt(K)), 2.46e-7
+// on the LDS GEMV that served it before.
+// bf16 8 x 11008 x 4096 19.4 us against 73.7 there, 8 x 16384 x 1024 16.5 against
+// 27, f32 8 x 11008 x 4096 38 (4.7 TB/s) against 97, 8 x 4096 x 4096 16 against 41.
+constexpr int kSkLongWaves = 8;
+constexpr int64_t kSkLongGrid = 1 << 22;  // workgroups per launch (2^31 threads)
+
+template <InType T, EpiKind E, int BLK>
+__global__ __launch_bounds__(kSkLongWaves * 64) void skinny_long(const GemvArgs g,
+                                                                 const EpiParams ep, int row0) {
+    constexpr int ROWS = 8 * BLK, NW = kSkLongWaves;
+    using Mm = Mma16<T>;
+    using acc_t = typename Mm::acc_t;
+    using val_t = typename Mm::val_t;
+    constexpr int esz = (T == InType::I8) ? 1 : (T == InType::BF16 ? 2 : 4);
+    __shared__ val_t comb[NW][BLK * 2 * 64];
+    const int64_t kb = ((int64_t)g.K * esz + 15) / 16 * 16;
+    const int nk = (int)((kb + kSkStep - 1) / kSkStep);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lg = lane >> 4;
+    const int chunk = 2 * lg + (li & 1);
+    const int kseg = (nk + NW - 1) / NW;
+    const int ks0 = wave * kseg, ks1 = ks0 + kseg < nk ? ks0 + kseg : nk;
+    const int64_t zb = blockIdx.y;
+    const int64_t ld_b = g.ld * esz, vld_b = g.vld * esz;
+    const int r0 = row0 + (int)blockIdx.x * ROWS;
+    const uint8_t *mat = (const uint8_t *)g.mat + zb * g.bsm * esz + (int64_t)r0 * ld_b;
+    const uint8_t *vec = (const uint8_t *)g.vec + zb * g.bsv * esz;
+    const int nrows = g.R - r0 < ROWS ? g.R - r0 : ROWS;
+    const uint32_t num = (uint32_t)((nrows - 1) * ld_b + kb);
+    const uint32_t vnum = (uint32_t)((g.nvec - 1) * vld_b + kb);
+    uint32_t off[BLK];
+#pragma unroll
+    for (int b = 0; b < BLK; ++b) off[b] = (uint32_t)((8 * b + (li >> 1)) * ld_b + 16 * chunk);
+    const uint32_t voff = (uint32_t)(li < g.nvec ? li : 0) * (uint32_t)vld_b + 32 * lg;
+    const uint32_t vout = (uint32_t)(li >= g.nvec) << 31;  // columns past nvec: zeros
+    // Chunks past K or the wave's range read zeros (bit 31 is past any extent here).
+    auto issue = [&](int s0, v4i_s (&m)[kSkPF][BLK], v4i_s (&x)[kSkPF][2]) {
+#pragma unroll
+        for (int p = 0; p < kSkPF; ++p) {
+            const int s = s0 + p;
+            const uint32_t k = (uint32_t)s * kSkStep;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const bool in = s < ks1 && (int64_t)k + 16 * (2 * lg + h) < kb;
+                x[p][h] = load16v(vec, vnum, (voff + k + 16 * h) | vout | (uint32_t)!in << 31);
+            }
+            const bool in = s < ks1 && (int64_t)k + 16 * chunk < kb;
+#pragma unroll
+            for (int b = 0; b < BLK; ++b)
+                m[p][b] = load16(mat, num, (off[b] + k) | (uint32_t)!in << 31);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    val_t sum[2][BLK][2] = {};  // [h][block][e]: the running sums of a matrix row's halves
+    auto run = [&](int s0, const v4i_s (&m)[kSkPF][BLK], const v4i_s (&x)[kSkPF][2]) {
+        acc_t acc[2][BLK] = {};
+#pragma unroll
+        for (int p = 0; p < kSkPF; ++p)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int b = 0; b < BLK; ++b) acc[h][b] = Mm::step(m[p][b], x[p][h], acc[h][b]);
+#pragma unroll
+        for (int b = 0; b < BLK; ++b)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                sum[0][b][e] += acc[0][b][2 * e];
+                sum[1][b][e] += acc[1][b][2 * e + 1];
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    v4i_s m0[kSkPF][BLK], m1[kSkPF][BLK], x0[kSkPF][2], x1[kSkPF][2];
+    if (ks0 < ks1) {
+        issue(ks0, m0, x0);
+        for (int s = ks0; s < ks1; s += 2 * kSkPF) {
+            if (s + kSkPF < ks1) issue(s + kSkPF, m1, x1);
+            run(s, m0, x0);
+            if (s + kSkPF >= ks1) break;
+            if (s + 2 * kSkPF < ks1) issue(s + 2 * kSkPF, m0, x0);
+            run(s + kSkPF, m1, x1);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < BLK; ++b)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) comb[wave][(b * 2 + e) * 64 + lane] = sum[0][b][e] + sum[1][b][e];
+    __syncthreads();
+    for (int x = tid; x < BLK * 2 * 64; x += NW * 64) {
+        val_t v = comb[0][x];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += comb[w][x];
+        const int b = x / 128, e = (x / 64) % 2, ln = x % 64;
+        const int row = r0 + 8 * b + 2 * (ln >> 4) + e, j = ln & 15;
+        if (j < g.nvec && row < g.R) Store<E>::apply(ep, zb, j, row, v);
+    }
+}
+
+template <InType T, EpiKind E>
+static hipError_t skinny_long_go(const GemvArgs &g, const EpiParams &ep, hipStream_t stream) {
+    const int cus = g.cus > 0 ? g.cus : 256;
+    const int64_t R = g.R, nb = g.batch;
+    const int rows = (R + 31) / 32 * nb >= cus ? 32 : ((R + 15) / 16 * nb >= cus ? 16 : 8);
+    const dim3 block(kSkLongWaves * 64);
+    for (int64_t r = 0; r < R; r += rows * kSkLongGrid) {
+        const int64_t items = (R - r + rows - 1) / rows;
+        const dim3 grid((unsigned)(items < kSkLongGrid ? items : kSkLongGrid), (unsigned)nb);
+        if (rows == 32)
+            hipLaunchKernelGGL((skinny_long<T, E, 4>), grid, block, 0, stream, g, ep, (int)r);
+        else if (rows == 16)
+            hipLaunchKernelGGL((skinny_long<T, E, 2>), grid, block, 0, stream, g, ep, (int)r);
+        else
+            hipLaunchKernelGGL((skinny_long<T, E, 1>), grid, block, 0, stream, g, ep, (int)r);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_skinny_long(InType in, const GemvArgs &g, const EpiParams &ep,
+                              hipStream_t stream) {
+    const int64_t esz = in == InType::I8 ? 1 : (in == InType::BF16 ? 2 : 4);
+    // (32-bit offsets from an item's first row and the first vector; 16-byte
+    // vector chunks)
+    if (g.nvec < 1 || g.nvec > 16 || g.R < 1 || g.ld < 0 || g.vld < 0 || g.vks != 1 ||
+        15 * g.vld * esz + g.K * esz >= 0x7FFFFF00ll || g.batch < 1 || g.batch > kMaxGridZ)
+        return hipErrorInvalidValue;
+    switch (in) {
+    case InType::I8:
+        if (ep.kind == EpiKind::I32) return skinny_long_go<InType::I8, EpiKind::I32>(g, ep, stream);
+        if (ep.kind == EpiKind::Q8) return skinny_long_go<InType::I8, EpiKind::Q8>(g, ep, stream);
+        break;
+    case InType::F32:
+        if (ep.kind == EpiKind::F32) return skinny_long_go<InType::F32, EpiKind::F32>(g, ep, stream);
+        break;
+    case InType::BF16:
+        if (ep.kind == EpiKind::F32) return skinny_long_go<InType::BF16, EpiKind::F32>(g, ep, stream);
+        if (ep.kind == EpiKind::BF16)
+            return skinny_long_go<InType::BF16, EpiKind::BF16>(g, ep, stream);
+        break;
+    }
+    return hipErrorInvalidValue;
+}
+
+bool skinny_is_long(InType in, int64_t K, int nvec) {
+    return skinny_lds_bytes(in, K, nvec) > kSkinnyLdsMax;
+}
+
 // ---- skinny_cols ------------------------------------------------------------
 // The same products with a matrix of unit row stride (element (r, p) at
 // r + p*mks, any mks and alignment; x * W with W row-major) and k-contiguous
@@ -489,7 +643,7 @@ struct SkCols<InType::I8> {
     }
 };
 
-template <InType T>
+template <InType T, bool LONG>
 __global__ __launch_bounds__(64) void skinny_cols(const GemvArgs g, int ranges) {
     using Sc = SkCols<T>;
     using elem_t = typename Sc::elem_t;
@@ -517,6 +671,20 @@ __global__ __launch_bounds__(64) void skinny_cols(const GemvArgs g, int ranges) 
                         (int64_t)(li < g.nvec ? li : g.nvec - 1) * g.vld + k0;
 
     typename Sc::acc_t acc[RPL] = {};
+    // LONG (floats): skinny_long's running sums, every kSkPF steps of the range.
+    typename Sc::acc_t sum[LONG ? RPL : 1] = {};
+    auto step = [&](int s, const v2i_s (&m)[EPC], v4i_s x) {
+        Sc::step(m, x, acc);
+        if constexpr (LONG) {
+            if ((s - ks0) % kSkPF == kSkPF - 1 || s == ks1 - 1) {
+#pragma unroll
+                for (int t = 0; t < RPL; ++t) {
+                    sum[t] += acc[t];
+                    acc[t] = typename Sc::acc_t{};
+                }
+            }
+        }
+    };
     // Two batches in turn, the next one's loads in flight while one is
     // multiplied.  All loads of a batch are issued before any is used; steps past
     // the end load the last one again and are left out.
@@ -533,7 +701,7 @@ __global__ __launch_bounds__(64) void skinny_cols(const GemvArgs g, int ranges) 
     auto mul = [&](int s, const v2i_s (&m)[PF][EPC], const v4i_s (&x)[PF]) {
 #pragma unroll
         for (int u = 0; u < PF; ++u)
-            if (s + u < kfull) Sc::step(m[u], x[u], acc);
+            if (s + u < kfull) step(s + u, m[u], x[u]);
         __builtin_amdgcn_sched_barrier(0);
     };
     if (ks0 < kfull) {
@@ -564,7 +732,7 @@ __global__ __launch_bounds__(64) void skinny_cols(const GemvArgs g, int ranges) 
         }
         v4i_s x;
         __builtin_memcpy(&x, v, 16);
-        Sc::step(m, x, acc);
+        step(whole, m, x);
     }
     if (li < g.nvec) {
         val_t *out = (val_t *)g.part + ((zb * 2 * ranges + unit) * g.nvec + li) * g.R;
@@ -572,7 +740,7 @@ __global__ __launch_bounds__(64) void skinny_cols(const GemvArgs g, int ranges) 
         for (int q = 0; q < 4; ++q) {
             val_t v[RPL];
 #pragma unroll
-            for (int t = 0; t < RPL; ++t) v[t] = acc[t][q];
+            for (int t = 0; t < RPL; ++t) v[t] = LONG ? sum[LONG ? t : 0][q] : acc[t][q];
             __builtin_memcpy(out + row_of(4 * lg + q), v, sizeof(v));
         }
     }
@@ -596,15 +764,15 @@ __global__ __launch_bounds__(64) void cols_sum(const GemvArgs g, const EpiParams
     Store<E>::apply(ep, zb, j, (int)r, sum);
 }
 
-// K ranges: 4 for floats (the row kernel's order); i8 up to 16 while that leaves
-// fewer than four waves per CU, a batch of loads to each and a scratch no larger
+// K ranges: the row kernel's for floats (its order); i8 up to 16 while that leaves
+// fewer than four waves per CU, half a batch of loads to each and a scratch no larger
 // than a quarter of the matrix.
 static int skinny_cols_ranges(InType in, int64_t R, int64_t K, int nvec, int64_t batch, int cus) {
+    if (in != InType::I8) return skinny_is_long(in, K, nvec) ? kSkLongWaves : kSkWaves;
     int ranges = 4;
-    if (in != InType::I8) return ranges;
     const int64_t groups = (R + 127) / 128 * batch;
     while (ranges < 16 && groups * 2 * ranges < 4 * (int64_t)(cus > 0 ? cus : 256) &&
-           K >= (int64_t)2 * ranges * 128 * SkCols<InType::I8>::PF &&
+           K >= (int64_t)ranges * 128 * SkCols<InType::I8>::PF &&
            4 * ranges * nvec * 4 * 4 <= K)
         ranges *= 2;
     return ranges;
@@ -619,15 +787,17 @@ static hipError_t skinny_cols_go(const GemvArgs &g, const EpiParams &ep, hipStre
     constexpr int ROWS = 16 * 8 / (T == InType::I8 ? 1 : (T == InType::BF16 ? 2 : 4));
     const int ranges = skinny_cols_ranges(T, g.R, g.K, g.nvec, g.batch, g.cus);
     const int64_t groups = ((int64_t)g.R + ROWS - 1) / ROWS;
-    hipLaunchKernelGGL((skinny_cols<T>), dim3((unsigned)(groups * 2 * ranges), (unsigned)g.batch),
-                       dim3(64), 0, stream, g, ranges);
+    const dim3 parts((unsigned)(groups * 2 * ranges), (unsigned)g.batch);
     const dim3 grid((unsigned)(((int64_t)g.R + 63) / 64), (unsigned)g.nvec, (unsigned)g.batch);
+    if (T != InType::I8 && ranges == kSkLongWaves)
+        hipLaunchKernelGGL((skinny_cols<T, T != InType::I8>), parts, dim3(64), 0, stream, g, ranges);
+    else
+        hipLaunchKernelGGL((skinny_cols<T, false>), parts, dim3(64), 0, stream, g, ranges);
     if constexpr (T == InType::I8) {
         if (ranges == 16)
             hipLaunchKernelGGL((cols_sum<T, E, 16>), grid, dim3(64), 0, stream, g, ep);
-        else if (ranges == 8)
-            hipLaunchKernelGGL((cols_sum<T, E, 8>), grid, dim3(64), 0, stream, g, ep);
     }
+    if (ranges == 8) hipLaunchKernelGGL((cols_sum<T, E, 8>), grid, dim3(64), 0, stream, g, ep);
     if (ranges == 4) hipLaunchKernelGGL((cols_sum<T, E, 4>), grid, dim3(64), 0, stream, g, ep);
     return hipGetLastError();
 }

@@ -25,7 +25,12 @@ def values(n, dt, seed, dev):
 # (i8) long enough for 8 and 16 ranges
 @pytest.mark.parametrize("shape", [(2, 1024, 17), (3, 1025, 33), (5, 1100, 64), (8, 2048, 1000),
                                    (9, 1536, 129), (16, 1984, 40), (4, 8200, 75), (2, 6144, 300),
-                                   (15, 1601, 2050), (2, 16384, 65), (4, 4095, 257)],
+                                   (15, 1601, 2050), (2, 16384, 65), (4, 4095, 257), (1, 8300, 70),
+                                   # vectors beyond the LDS: one row group, 8-, 16- and
+                                   # 32-row ones, K ending inside a step and a chunk,
+                                   # more than eight vectors
+                                   (8, 16385, 40), (5, 14008, 2049), (8, 8190, 4100),
+                                   (7, 9300, 8200), (16, 4104, 2048), (12, 5503, 2100)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_unit_row_stride_equals_k_contiguous(dev, dtype, shape):
     m, k, n = shape
@@ -51,7 +56,7 @@ def test_unit_row_stride_equals_k_contiguous(dev, dtype, shape):
             f(m, k, n, alpha, x, rsa, csa, b, rsb, csb, beta, c, n, 1, b_off=bo)
             outs.append(c)
         # the transposed product: W^T (n x k, column-major) times the vectors
-        c = c0.view(m, n).T.contiguous().reshape(-1)
+        c = c0.view(m, n).T.clone(memory_format=torch.contiguous_format).reshape(-1)
         f(n, k, m, alpha, w, 1, n, a, 1, k, beta, c, m, 1)
         outs.append(c.view(n, m).T.contiguous().reshape(-1))
         for c in outs[1:]:
