@@ -1,5 +1,5 @@
 // f32x.hip -- f32 GEMM on the bf16 matrix cores, at f32 precision: every operand
-// element is split into three bf16 parts and six of the nine products of parts
+// element is split into three bf16 parts and eight of the nine products of parts
 // are summed in f32.
 //
 // Replaces the same layers as mma_kernel.h (src/driver.rs:402-944,
@@ -7,20 +7,27 @@
 // small products of small.hip.
 //
 // Why.  CDNA4's f32 matrix rate is 1/16 of its bf16 rate (157 against 2500
-// TFLOP/s), so six bf16 products per f32 product leave 2.6 times the f32 rate.
+// TFLOP/s), so eight bf16 products per f32 product leave twice the f32 rate.
 // The split loses nothing: a = h + m + l with h = bf16(a), m = bf16(a - h),
 // l = a - h - m is exact (24 significant bits in three times eight, both
-// subtractions exact), the six products hh, hm, mh, mm, hl, lh are exact in f32
-// pairs of 8-bit significands, and the three left out (ml, lm, ll) are below
-// 2^-26 of |a||b| together.  The running sum is rounded six times per 32 k, once
-// per product of parts, where the f32 instructions round it at least 16 times;
-// with HL (the shapes small.hip would serve, whose sixteen partial sums round
-// less) the five small products, 2^-8 of hh, have accumulators of their own and
-// the large sum is rounded once per 32 k.
-// Measured (row-major, against the f32 tiles with B packed first): 2048^3 88.4 us =
-// 194 TFLOP/s against 140.1, relative error 4.9e-7 against 8.1e-7; 1024^3 22 against
-// 35; 488 x 3136 x 2512 75.6 against 102.8.  Bound by the matrix cores at the
-// clock the chip's power limit leaves them: 78 us on zeros.
+// subtractions exact), and the products of parts are exact in f32 (pairs of 8-bit
+// significands).  |m| <= 2^-8 |a| and |l| <= 2^-17 |a|, so the one product left
+// out (ll) is at most 2^-34 of |a||b|.
+//
+// Sums.  The matrix cores cut the lower of two addends off at the result's last
+// bit, so a small product added to a sum there costs up to an ulp.  The seven
+// small products (2^-7 of the whole at most) of 32 k are therefore summed apart,
+// smallest first, and added to the sum, which has taken the large ones (hh), in
+// one rounded f32 addition: a sum of a single term is its correctly rounded value
+// but within 2^-6 ulp of a tie (the f32 instructions': always).  With HL (the shapes
+// small.hip would serve, whose sixteen partial sums round less) the small sum
+// runs over all of K and is added once.  With ml and lm left out too, together up
+// to 2^-24, and all products in one sum a single term erred by up to 1.4 ulp
+// (2048^3: 95 us instead of 112).
+// Measured (row-major, against the f32 tiles with B packed first): 2048^3 112 us =
+// 153 TFLOP/s against 138, relative error on normal inputs 2.1e-7 against 8.1e-7;
+// 1024^3 22.7 against 29.2, 1.5e-7 against 5.7e-7; 488 x 3136 x 2512 78 against 95.
+// Bound by the matrix cores at the clock the chip's power limit leaves them.
 //
 // The split needs every part to be a normal bf16 number: |a| below the largest
 // bf16, and 0 or at least 2^-102.  A tile watches for the rest: the smallest
@@ -92,7 +99,7 @@ __device__ __forceinline__ void x_split(const float (&v)[8], v4u_x &h, v4u_x &m,
 
 // AK / BK: the operand is k-contiguous.
 constexpr int kXThreads = 512, kXGroup = 256;
-// HL: the five small products in accumulators of their own.
+// HL: the small products in accumulators of their own over all of K.
 template <int BM, int BN, bool AK, bool BK, bool HL>
 __global__ __launch_bounds__(kXThreads)
 __attribute__((amdgpu_waves_per_eu(BM == 64 ? 4 : 2, BM == 64 ? 4 : 2)))
@@ -219,32 +226,51 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
             if (o < TM) a[p][o < TM ? o : 0] = v; else b[p][o < TM ? 0 : o - TM] = v;
         }
     };
-    v4f_x acc[TM][TN] = {}, low[HL ? TM : 1][HL ? TN : 1] = {};
-    // Smallest products first; the blocks of a step are independent.  From the
-    // third step on, a chunk of the group's next stage is split beside each
-    // step's MFMAs (a wave issues three VALU instructions while one runs).
+    v4f_x acc[TM][TN] = {};
+    // Four blocks at a time: their large products into the sums, then the small
+    // ones, smallest first, into four accumulators that start from zero and are
+    // added to the sums behind the next four blocks' large products (by when the
+    // last of them has left the matrix cores).  The group's next stage is split
+    // beside the small products, a chunk of it at a time (a wave issues three VALU
+    // instructions while one MFMA runs).
+    constexpr int NB = TM * TN, NQ = NB / 4;
+    static_assert(NB % 4 == 0 && (NQ == NC || NQ == 1) && !(HL && NQ != 1), "blocks");
+    v4f_x t[4] = {};
+    auto add = [&](int q) {
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[(4 * q + y) / TN][(4 * q + y) % TN] += t[y];
+        __builtin_amdgcn_sched_barrier(0);
+    };
     auto mul = [&]() {
-        constexpr int kPart[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+        constexpr int kSmall = 7;
+        constexpr int kPart[kSmall][2] = {{2, 1}, {1, 2}, {2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
 #pragma unroll
-        for (int s = 0; s < 6; ++s) {
+        for (int q = 0; q < NQ; ++q) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+            for (int y = 0; y < 4; ++y) {
+                const int i = (4 * q + y) / TN, j = (4 * q + y) % TN;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[0][j], a[0][i], acc[i][j], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (q > 0) add(q - 1);
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    v4f_x &c = HL && s < 5 ? low[HL ? i : 0][HL ? j : 0] : acc[i][j];
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[kPart[s][0]][j],
-                                                                a[kPart[s][1]][i], c, 0, 0, 0);
+            for (int s = 0; s < kSmall; ++s)
+#pragma unroll
+                for (int y = 0; y < 4; ++y) {
+                    const int i = (4 * q + y) / TN, j = (4 * q + y) % TN;
+                    t[y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        b[kPart[s][0]][j], a[kPart[s][1]][i], s == 0 && !HL ? v4f_x{0, 0, 0, 0} : t[y], 0, 0, 0);
                 }
-            if (s >= 6 - NC) {
-                split(s - (6 - NC));
 #pragma unroll
-                for (int x = 0; x < TM * TN; ++x) {
-                    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 56 / (TM * TN) + 1, 0);
-                }
+            for (int c = 0; c < NC / NQ; ++c) split(q * (NC / NQ) + c);
+#pragma unroll
+            for (int x = 0; x < 4 * kSmall; ++x) {
+                __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, NQ == 1 ? 4 : 3, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (!HL) add(NQ - 1);
     };
     // Ends a slot: this wave's LDS reads and writes are done, then the barrier
     // (loads of later stages stay in flight across it).  The scheduling barriers
@@ -313,14 +339,7 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
         slot_end();
     }
 
-    if constexpr (HL) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[i][j][q] += low[i][j][q];
-    }
+    if constexpr (HL) add(0);
     // Which 64 x 64 blocks have to be computed again.
 #pragma unroll
     for (int i = 0; i < NC; ++i)

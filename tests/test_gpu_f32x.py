@@ -43,8 +43,9 @@ def test_precision(dev, m, k, n, la, lb, pad):
     c = c0.clone()
     gk.gemm_unchecked(m, k, n, 0.75, ab, rsa, csa, bb, rsb, csb, -1.25, c, n, 1)
     want = 0.75 * (a.double() @ b.double()) - 1.25 * c0.double().view(m, n)
-    # |error| <= roundings * u * sum |terms|: at most 6 per 32 k in each of two
-    # groups' sums, the split's 2^-26 and the four of the epilogue
+    # |error| <= roundings * u * sum |terms|: one per product of parts, 8 per 32 k
+    # in each of two groups' sums, which take every other 32 k; the product left out
+    # (2^-34) and the four of the epilogue
     u = 2.0 ** -24
     terms = 0.75 * (a.abs().double() @ b.abs().double()) + 1.25 * c0.abs().double().view(m, n)
     roundings = 6 * ((k + 31) // 32) + 6
@@ -57,6 +58,31 @@ def test_precision(dev, m, k, n, la, lb, pad):
     p = torch.zeros(m * n, device=dev)
     gk.gemm_unchecked(m, k, n, 1.0, ab, rsa, csa, bb, rsb, csb, 0.0, p, n, 1)
     assert torch.equal(f.view(m, n), torch.relu(p.view(m, n) + bias))
+
+
+# rows of 64 x 64 and 128 x 128 tiles, with (600 x 700) and without accumulators of
+# their own for the small products
+@pytest.mark.parametrize("m,k,n", [(600, 128, 700), (1030, 129, 1000), (2049, 160, 2047)])
+def test_sums_of_one_term_are_correctly_rounded(dev, m, k, n):
+    """One nonzero per row of A: every output is one product, which the f32
+    instructions round correctly.  Here the product of parts left out is below
+    2^-34 of it, and the small ones' sum, 2^-7 of it, loses up to 2^-30 of it in each
+    of its last two additions (its others are far smaller): with the last, rounded
+    one half an ulp and 2^-6 ulp; 2^-5 allowed."""
+    b = randn(k * n, 31, dev).view(k, n)
+    v = randn(m, 32, dev)
+    # the largest m and l against h, alike in sign: 1 + 2^-8 - 2^-17
+    worst = torch.tensor(0x3F807FC0, dtype=torch.int32).view(torch.float32).item()
+    b[:, ::7], v[::5] = worst, worst
+    at = torch.arange(m, device=dev) * 37 % k
+    a = torch.zeros(m, k, device=dev)
+    a[torch.arange(m, device=dev), at] = v
+    c = torch.zeros(m * n, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, a.view(-1), k, 1, b.reshape(-1), n, 1, 0.0, c, n, 1)
+    want = v.double()[:, None] * b[at].double()
+    ulp = 2.0 ** (torch.frexp(want).exponent.double() - 24)
+    err = ((c.view(m, n).double() - want) / ulp).abs()
+    assert err.max() <= 0.5 + 2.0 ** -5, err.max()
 
 
 def special(m, k, n, seed, dev):
