@@ -1118,7 +1118,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         const int64_t kc = round_up64((k + splits - 1) / splits, 64 / (int64_t)esz);
         splits = (int)((k + kc - 1) / kc);
     }
-    // f32 routes, operands read in place (no pack), by the element shape only so
+    // f32 routes, operands read in place, by the element shape only so
     // that a batched element takes the route of its standalone product:
     //  * small_f32: products that would split K (too few 64 x 64 tiles for the
     //    CUs) in one launch, a workgroup per 32 x 32 block with K split over its 16
@@ -1143,8 +1143,30 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         if (k >= kF32xMinK && f32x_fits(M, N) &&
             (splits == 1 || (small_f32_enabled() && blocks > cus &&
                              (blocks + cus - 1) / cus * ((k + 31) / 32) <= 256))) {
+            // Every tile row or column reads an operand again, a cache line for a few
+            // elements where neither of its strides is short: such an operand is packed
+            // first (the sums do not depend on it).  2048^3 with every second column of
+            // A 181 us in place, 125 packed (f32 tiles: 146), also of B^T's rows 267 and
+            // 131 (148); 1000 x 300 x 1100 30 and 21 (23), 53 and 26 (24).  Rows two
+            // apart stay in place: 126 (146), 17 (24); four apart in A, two in B 151
+            // (153), 64 on 3000 x 130 x 3000 (59).
+            auto in_place = [](const Opnd &o) { return o.ks == 1 || (o.rs >= 0 && o.rs <= 2); };
+            const size_t pa = in_place(A) ? 0 : pack_bytes(in, M, k, batch, A);
+            const size_t pb = in_place(Bt) ? 0 : pack_bytes(in, N, k, batch, Bt);
+            if (pa + pb > 0) {
+                uint8_t *dst = nullptr;
+                if (const int r = region_get(rg, pa + pb, &dst)) return r;
+                PackJob jobs[2];
+                int nj = 0;
+                if (pa) jobs[nj++] = pack_job(in, &A, M, k, batch, dst);
+                if (pb) jobs[nj++] = pack_job(in, &Bt, N, k, batch, dst + pa);
+                const hipError_t e = launch_pack(in, jobs, nj, tl_stream);
+                if (e != hipSuccess) return hip_fail(e, "pack");
+            }
+            const SmallArgs xa{A.p, Bt.p, A.rs, A.ks, Bt.rs, Bt.ks, A.bs, Bt.bs,
+                               (int32_t)M, (int32_t)N, (int32_t)k, (int32_t)batch};
             ep.vec4 = ep.csc == 1;
-            hipError_t e = launch_f32x(sa, ep, splits > 1, g_num_cus, tl_stream);
+            hipError_t e = launch_f32x(xa, ep, splits > 1, g_num_cus, tl_stream);
             if (e != hipSuccess) return hip_fail(e, "f32 gemm launch");
             return finish("f32 gemm");
         }

@@ -85,6 +85,32 @@ def test_sums_of_one_term_are_correctly_rounded(dev, m, k, n):
     assert err.max() <= 0.5 + 2.0 ** -5, err.max()
 
 
+@pytest.mark.parametrize("m,k,n", [(600, 150, 700), (1300, 131, 900)])
+@pytest.mark.parametrize("rs,ks,packed", [
+    (1, 1500, False), (2, 3100, False), (3, 4600, True), (0, 1, False), (700, 1, False),
+    (1500, 2, True), (700, -1, True), (-700, 1, False), (-1, 1500, True), (5, 7600, True),
+    (3000, 4, True), (0, 3, False)])
+def test_operand_strides(dev, m, k, n, rs, ks, packed):
+    """Any strides of either operand: the bits of the call on row-major copies.  An
+    operand without a short stride, which every tile would read a cache line per
+    element, is packed into the workspace; others are read in place."""
+    def operand(rows, seed):
+        lo = min(0, rs * (rows - 1)) + min(0, ks * (k - 1))
+        hi = max(0, rs * (rows - 1)) + max(0, ks * (k - 1))
+        buf = randn(hi - lo + 1, seed, dev)
+        at = torch.arange(rows, device=dev)[:, None] * rs + torch.arange(k, device=dev)[None] * ks
+        return buf, -lo, buf[at - lo]
+
+    a, a0, ac = operand(m, 61)
+    b, b0, bc = operand(n, 62)  # B^T
+    want, got = torch.zeros(m * n, device=dev), torch.zeros(m * n, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, ac.reshape(-1), k, 1, bc.reshape(-1), 1, k, 0.0, want, n, 1)
+    ws = gk.Workspace()
+    gk.gemm_unchecked(m, k, n, 1.0, a, rs, ks, b, ks, rs, 0.0, got, n, 1, ws=ws, a_off=a0, b_off=b0)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    assert (ws.bytes() > 0) == packed
+
+
 def special(m, k, n, seed, dev):
     """A and B with an infinity, a NaN, the largest f32, subnormals and rows of
     magnitudes whose split would leave the bf16 range."""
