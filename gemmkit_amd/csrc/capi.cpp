@@ -842,6 +842,13 @@ int region_get(const Region &rg, size_t bytes, uint8_t **out) {
     return GK_OK;
 }
 
+// Whether region_get can give `bytes`: not beyond a fixed region, nor by growing the
+// arena under graph capture.  For scratch that only makes a call faster.
+bool region_fits(const Region &rg, size_t bytes) {
+    if (rg.fixed) return bytes <= rg.fixed_bytes;
+    return resolve_ws(rg.ws)->bytes >= bytes || !stream_capturing();
+}
+
 int64_t out_size(EpiKind kind) {
     return kind == EpiKind::Q8 ? 1 : (kind == EpiKind::BF16 ? 2 : 4);
 }
@@ -1153,7 +1160,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
             auto in_place = [](const Opnd &o) { return o.ks == 1 || (o.rs >= 0 && o.rs <= 2); };
             const size_t pa = in_place(A) ? 0 : pack_bytes(in, M, k, batch, A);
             const size_t pb = in_place(Bt) ? 0 : pack_bytes(in, N, k, batch, Bt);
-            if (pa + pb > 0) {
+            if (pa + pb > 0 && region_fits(rg, pa + pb)) {
                 uint8_t *dst = nullptr;
                 if (const int r = region_get(rg, pa + pb, &dst)) return r;
                 PackJob jobs[2];

@@ -111,6 +111,26 @@ def test_operand_strides(dev, m, k, n, rs, ks, packed):
     assert (ws.bytes() > 0) == packed
 
 
+def test_strided_operand_under_capture(dev):
+    """The pack is only for speed: with a workspace that capture cannot grow the
+    operand is read in place, and the replays give the same bits."""
+    m, k, n = 600, 150, 700
+    a, b = randn(2 * m * k, 71, dev), randn(k * n, 72, dev)
+    want, got = torch.zeros(m * n, device=dev), torch.zeros(m * n, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, a, 2 * k, 2, b, n, 1, 0.0, want, n, 1)
+    ws = gk.Workspace()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gk.gemm_unchecked(m, k, n, 1.0, a, 2 * k, 2, b, n, 1, 0.0, got, n, 1, ws=ws)
+    assert ws.bytes() == 0
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
 def special(m, k, n, seed, dev):
     """A and B with an infinity, a NaN, the largest f32, subnormals and rows of
     magnitudes whose split would leave the bf16 range."""
