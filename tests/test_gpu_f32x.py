@@ -121,8 +121,12 @@ def test_strided_operand_under_capture(dev):
     ws = gk.Workspace()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        gk.gemm_unchecked(m, k, n, 1.0, a, 2 * k, 2, b, n, 1, 0.0, got, n, 1, ws=ws)
+    gk.set_synchronous(False)
+    try:
+        with torch.cuda.graph(graph):
+            gk.gemm_unchecked(m, k, n, 1.0, a, 2 * k, 2, b, n, 1, 0.0, got, n, 1, ws=ws)
+    finally:
+        gk.set_synchronous(True)
     assert ws.bytes() == 0
     for _ in range(3):
         got.zero_()
