@@ -29,14 +29,21 @@
 // 1024^3 22.7 against 29.2, 1.5e-7 against 5.7e-7; 488 x 3136 x 2512 78 against 95.
 // Bound by the matrix cores at the clock the chip's power limit leaves them.
 //
-// The split needs every part to be a normal bf16 number: |a| below the largest
-// bf16, and 0 or at least 2^-102.  A tile watches for the rest: the smallest
-// nonzero magnitude of each 64-row panel of A and B while it is split, and any
-// accumulator that is not finite (an infinite or NaN input, or one that rounds
-// to an infinite h, always leaves one).  A 64 x 64 block of the output that
-// such a panel or accumulator touches is computed again with the f32
-// instructions from memory.  The blocks are cut at multiples of 64 whatever
-// the tile, so an element's value does not depend on the tile that computed it.
+// Range.  Elements are scaled by 2^23 as they are split and the sums by 2^-46 at
+// the end, both exact (a subnormal result is rounded once more): every part of
+// every finite f32 below 2^105 is then a normal bf16 number or 0 (f32 values are
+// multiples of 2^-149, so parts of 2^-126), and every product of parts that
+// matters to a result of 2^-149 or more is a normal f32.  Larger elements,
+// infinities and NaN leave a sum that is not finite, and so do results of 2^82 or
+// more: a 16 x 16 block of the output with such a sum is computed again with the
+// f32 instructions.  The blocks are cut at multiples of 16 whatever the tile, so an
+// element's value does not depend on the tile that computed it.
+// The second pass waits for the first and shares no operands between waves:
+// 2048^3 with an infinity among 100,000 elements 280 us, with one in every block 360,
+// against 108 without and 138 on the f32 tiles; zeros, subnormals and the smallest
+// normal values cost nothing (unscaled parts below 2^-126 sent 64 x 64 blocks to
+// such a pass: 380 us on 2048^3, 110 against 22 on 1024^3, with one element of
+// 10,000 at 1e-35).
 //
 // Schedule.  One workgroup of two groups of four waves per BM x BN tile; a stage
 // is 32 k, group g multiplies the stages of its parity (every wave of it a
@@ -71,14 +78,8 @@ typedef __bf16 v8bf_x __attribute__((ext_vector_type(8)));
 
 constexpr int kXStage = 32;              // k per stage
 constexpr int kXRow = kXStage * 2;       // LDS bytes of a row of one part
-// 2 * (bits of 2^-102) - 1: see x_watch.
-constexpr uint32_t kXTiny = ((uint32_t)(127 - 102) << 24) - 1;
-
-// Smallest nonzero |a| seen, as 2*|bits| - 1 (a zero becomes the largest).
-__device__ __forceinline__ uint32_t x_watch(uint32_t t, float a) {
-    const uint32_t v = (__float_as_uint(a) << 1) - 1u;
-    return v < t ? v : t;
-}
+// Both operands are scaled by 2^23 as they are split, the sums by 2^-46 at the end.
+constexpr float kXScale = 0x1p23f, kXUnscale = 0x1p-46f;
 
 // The three bf16 parts of 8 consecutive k of a row.  (Forming the differences
 // with v_dot2_f32_bf16, two instructions fewer per pair, doubled the time of a
@@ -86,7 +87,7 @@ __device__ __forceinline__ uint32_t x_watch(uint32_t t, float a) {
 __device__ __forceinline__ void x_split(const float (&v)[8], v4u_x &h, v4u_x &m, v4u_x &l) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float a0 = v[2 * i], a1 = v[2 * i + 1];
+        const float a0 = v[2 * i] * kXScale, a1 = v[2 * i + 1] * kXScale;
         const uint32_t hp = bf16x2_rne(a0, a1);
         const float r0 = a0 - __uint_as_float(hp << 16);
         const float r1 = a1 - __uint_as_float(hp & 0xFFFF0000u);
@@ -100,9 +101,10 @@ __device__ __forceinline__ void x_split(const float (&v)[8], v4u_x &h, v4u_x &m,
 // AK / BK: the operand is k-contiguous.
 constexpr int kXThreads = 512, kXGroup = 256;
 // HL: the small products in accumulators of their own over all of K.
-template <int BM, int BN, bool AK, bool BK, bool HL>
+// WPE: waves per SIMD (128 registers each at 4, 256 at 2).
+template <int BM, int BN, bool AK, bool BK, bool HL, int WPE>
 __global__ __launch_bounds__(kXThreads)
-__attribute__((amdgpu_waves_per_eu(BM == 64 ? 4 : 2, BM == 64 ? 4 : 2)))
+__attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void f32x_kernel(const SmallArgs g, const EpiParams ep) {
     constexpr int WTM = BM / 2, WTN = BN / 2;        // a wave's rows and columns
     constexpr int TM = WTM / 16, TN = WTN / 16;
@@ -110,10 +112,8 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
     static_assert(IA >= 1 && IB >= 1 && 64 % WTM == 0 && 64 % WTN == 0, "tile");
     constexpr int PART = (BM + BN) * kXRow;          // one part of one stage
     constexpr int BUF = 3 * PART;
-    constexpr int NPA = BM / 64, NPB = BN / 64;
     static_assert(kXThreads * TM * TN * 2 * 4 <= 3 * BUF, "exchange of the partial tiles");
     __shared__ __attribute__((aligned(16))) uint8_t lds[3 * BUF];
-    __shared__ int flags[NPA + NPB + NPA * NPB];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -127,7 +127,6 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
     const int m0 = tm * BM, n0 = tn * BN;
     const float *A = (const float *)g.a + zb * g.bsa;
     const float *B = (const float *)g.b + zb * g.bsb;
-    if (tid < NPA + NPB + NPA * NPB) flags[tid] = 0;
 
     // A thread's NC chunks of a stage, IA of A and the others of B: a row and eight
     // k, chunk c holding k 4c..4c+3 and 16+4c..16+4c+3 (both operands alike, so any
@@ -147,13 +146,11 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
         return kc_of(i) ? c % 4 : c / (of_a(i) ? BM : BN);
     };
     const float *src[NC];
-    uint32_t least[NC];    // x_watch
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         const int r = row_of(i), c = chunk_of(i);
         const int64_t o = of_a(i) ? (m0 + r < g.M ? m0 + r : g.M - 1) : (n0 + r < g.N ? n0 + r : g.N - 1);
         src[i] = (of_a(i) ? A + o * g.rsa : B + o * g.rsb) + 4 * c * ks_of(i);
-        least[i] = 0xFFFFFFFFu;
     }
     // LDS byte offset of a chunk in a part: rows 64 further down keep their slot
     // (k-contiguous), chunks two further on flip one bit of it.
@@ -197,11 +194,9 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
         }
     };
     auto split = [&](int i) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) least[i] = x_watch(least[i], raw[i][e]);
         x_split(raw[i], ph[i], pm[i], pl[i]);
         // (keeps the splitting in its slot: the compiler sinks it to the writes)
-        asm volatile("" : "+v"(ph[i]), "+v"(pm[i]), "+v"(pl[i]), "+v"(least[i]));
+        asm volatile("" : "+v"(ph[i]), "+v"(pm[i]), "+v"(pl[i]));
     };
     auto put = [&](uint8_t *buf, int i) {
         *(v4u_x *)(buf + dst(i)) = ph[i];
@@ -340,10 +335,6 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
     }
 
     if constexpr (HL) add(0);
-    // Which 64 x 64 blocks have to be computed again.
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-        if (least[i] < kXTiny) atomicOr(&flags[(of_a(i) ? 0 : NPA) + row_of(i) / 64], 1);
     // The groups exchange halves of their partial tiles: group 0 keeps rows
     // blocks [0, TM/2) of each wave's part, group 1 the others.
     constexpr int TH = TM / 2;
@@ -355,53 +346,86 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
             ex[(i * TN + j) * kXThreads + tid] = grp == 0 ? acc[TH + i][j] : acc[i][j];
     __syncthreads();
     v4f_x out[TH][TN];
-    bool odd = false;
+    unsigned odd = 0;  // blocks with a sum that is not finite, one bit each
 #pragma unroll
     for (int i = 0; i < TH; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const v4f_x o = ex[(i * TN + j) * kXThreads + (tid ^ kXGroup)];
             const v4f_x mine = grp == 0 ? acc[i][j] : acc[TH + i][j];
+            bool bad = false;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                out[i][j][q] = mine[q] + o[q];
-                odd = odd || (__float_as_uint(out[i][j][q]) & 0x7F800000u) == 0x7F800000u;
+                const float v = mine[q] + o[q];
+                bad = bad || (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u;
+                out[i][j][q] = v * kXUnscale;
             }
+            odd |= (unsigned)(__builtin_amdgcn_ballot_w64(bad) != 0) << (i * TN + j);
         }
-    const int ba = wm * WTM / 64, bb = wn * WTN / 64;
-    if (odd) atomicOr(&flags[NPA + NPB + ba * NPB + bb], 1);
-    __syncthreads();
     const int mw = m0 + wm * WTM + grp * TH * 16, nw = n0 + wn * WTN;
-    if (flags[ba] | flags[NPA + bb] | flags[NPA + NPB + ba * NPB + bb]) {
-        // v_mfma_f32_16x16x4_f32 on operands from memory, ascending k.
-        const float *ar[TH], *br[TN];
+    if (odd) {
+        // Those blocks again on v_mfma_f32_16x16x4_f32, operands from memory, 16 k
+        // a step (lane group c takes k 4c..4c+3 of it, one per instruction), the
+        // next step's loads in flight beside one's products.
+        constexpr int ND = TH + TN;
+        const float *p[ND];
 #pragma unroll
-        for (int i = 0; i < TH; ++i) {
-            const int64_t m = mw + 16 * i + fr < g.M ? mw + 16 * i + fr : g.M - 1;
-            ar[i] = A + m * g.rsa;
+        for (int d = 0; d < ND; ++d) {
+            const int64_t r = (d < TH ? mw + 16 * d : nw + 16 * (d - TH)) + fr;
+            p[d] = d < TH ? A + (r < g.M ? r : g.M - 1) * g.rsa : B + (r < g.N ? r : g.N - 1) * g.rsb;
         }
+        const int wsteps = g.K / 16;
+        auto fetch = [&](int t, float (&v)[ND][4]) {  // past the last whole step, that step again
+            const int64_t k = (int64_t)(t < wsteps ? t : wsteps - 1) * 16 + 4 * fc;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int64_t n = nw + 16 * j + fr < g.N ? nw + 16 * j + fr : g.N - 1;
-            br[j] = B + n * g.rsb;
+            for (int d = 0; d < ND; ++d) {
+                if (d < TH ? AK : BK) {
+                    const v4f_x x = *(const v4f_xu *)(p[d] + k);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[d][e] = x[e];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[d][e] = p[d][(k + e) * (d < TH ? g.ksa : g.ksb)];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        v4f_x again[TH][TN] = {};
+        auto mul4 = [&](const float (&v)[ND][4]) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TH; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        again[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[TH + j][e], v[i][e],
+                                                                           again[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        float v0[ND][4], v1[ND][4];
+        if (wsteps > 0) fetch(0, v0);
+        for (int t = 0; t < wsteps; t += 2) {
+            fetch(t + 1, v1);
+            mul4(v0);
+            if (t + 1 >= wsteps) break;
+            fetch(t + 2, v0);
+            mul4(v1);
+        }
+        if (g.K % 16 != 0) {  // the last, zeros past K
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int64_t k = (int64_t)wsteps * 16 + 4 * fc + e;
+                    v0[d][e] = k < g.K ? p[d][k * (d < TH ? g.ksa : g.ksb)] : 0.0f;
+                }
+            mul4(v0);
         }
 #pragma unroll
         for (int i = 0; i < TH; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) out[i][j] = v4f_x{0, 0, 0, 0};
-        for (int64_t k = 0; k < g.K; k += 4) {
-            const int64_t kk = k + fc;
-            float av[TH], bv[TN];
-#pragma unroll
-            for (int i = 0; i < TH; ++i) av[i] = kk < g.K ? ar[i][kk * g.ksa] : 0.0f;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) bv[j] = kk < g.K ? br[j][kk * g.ksb] : 0.0f;
-#pragma unroll
-            for (int i = 0; i < TH; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    out[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j], av[i], out[i][j], 0, 0, 0);
-        }
+            for (int j = 0; j < TN; ++j)
+                if (odd >> (i * TN + j) & 1) out[i][j] = again[i][j];
     }
 #pragma unroll
     for (int i = 0; i < TH; ++i) {
@@ -424,20 +448,20 @@ void f32x_kernel(const SmallArgs g, const EpiParams ep) {
     }
 }
 
-template <int BM, int BN, bool HL>
+template <int BM, int BN, bool HL, int WPE>
 static hipError_t f32x_go(const SmallArgs &g, const EpiParams &ep, hipStream_t stream) {
     const int64_t tiles = ((int64_t)(g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
     if (tiles * kXThreads > UINT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tiles, (unsigned)g.batch), block(kXThreads);
     const bool ak = g.ksa == 1, bk = g.ksb == 1;
     if (ak && bk)
-        hipLaunchKernelGGL((f32x_kernel<BM, BN, true, true, HL>), grid, block, 0, stream, g, ep);
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, true, true, HL, WPE>), grid, block, 0, stream, g, ep);
     else if (ak)
-        hipLaunchKernelGGL((f32x_kernel<BM, BN, true, false, HL>), grid, block, 0, stream, g, ep);
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, true, false, HL, WPE>), grid, block, 0, stream, g, ep);
     else if (bk)
-        hipLaunchKernelGGL((f32x_kernel<BM, BN, false, true, HL>), grid, block, 0, stream, g, ep);
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, false, true, HL, WPE>), grid, block, 0, stream, g, ep);
     else
-        hipLaunchKernelGGL((f32x_kernel<BM, BN, false, false, HL>), grid, block, 0, stream, g, ep);
+        hipLaunchKernelGGL((f32x_kernel<BM, BN, false, false, HL, WPE>), grid, block, 0, stream, g, ep);
     return hipGetLastError();
 }
 
@@ -458,10 +482,15 @@ hipError_t launch_f32x(const SmallArgs &g, const EpiParams &ep, bool fine, int c
     auto rounds = [&](int64_t t) {
         return (((g.M + t - 1) / t) * ((g.N + t - 1) / t) * g.batch + c - 1) / c;
     };
-    if (fine) return f32x_go<64, 64, true>(g, ep, stream);
+    // `fine` tiles of one round are alone on their CU and take the registers of two
+    // waves per SIMD (with four, the loop's addresses go through scratch memory:
+    // 2200 x 800 x 130 with A column-major 24.6 us against 17.7).
+    if (fine)
+        return rounds(64) == 1 ? f32x_go<64, 64, true, 2>(g, ep, stream)
+                               : f32x_go<64, 64, true, 4>(g, ep, stream);
     if (16 * rounds(128) <= 5 * rounds(64))
-        return f32x_go<128, 128, false>(g, ep, stream);
-    return f32x_go<64, 64, false>(g, ep, stream);
+        return f32x_go<128, 128, false, 2>(g, ep, stream);
+    return f32x_go<64, 64, false, 4>(g, ep, stream);
 }
 
 }  // namespace gk

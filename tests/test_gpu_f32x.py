@@ -1,6 +1,6 @@
 """f32 products on the bf16 matrix cores (f32x.hip): f32 precision over layouts,
-ragged sides and K tails, with and without the epilogue's terms; values the
-split cannot represent (infinities, NaN, the largest and the smallest
+ragged sides and K tails, with and without the epilogue's terms, and over the
+exponents; values the split cannot represent (infinities, NaN, the largest
 magnitudes); and the same bits from either tile, so from a batch and from its
 elements alone."""
 import pytest
@@ -137,7 +137,7 @@ def test_strided_operand_under_capture(dev):
 
 def special(m, k, n, seed, dev):
     """A and B with an infinity, a NaN, the largest f32, subnormals and rows of
-    magnitudes whose split would leave the bf16 range."""
+    magnitudes whose unscaled parts would leave the bf16 range."""
     a, b = randn(m * k, seed, dev).view(m, k), randn(k * n, seed + 1, dev).view(k, n)
     a[3, 5] = float("inf")
     a[m // 2, 7] = float("nan")
@@ -164,6 +164,43 @@ def test_values_outside_the_split(dev, m, k, n):
     # one rounding per k at most (the f32 instructions), and the subnormal grid
     bound = (k + 4) * (2.0 ** -24 * terms + 2.0 ** -149)
     assert ((got - want).abs()[ok] <= bound[ok]).all()
+
+
+@pytest.mark.parametrize("m,k,n", [(600, 150, 500), (1400, 131, 1300)])
+def test_precision_over_the_exponents(dev, m, k, n):
+    """Rows of A and columns of B from the smallest subnormals to 2^100: parts and
+    products of parts below the smallest normal numbers, results over all of f32."""
+    ea = torch.arange(m, device=dev) * 53 % 251 - 150
+    eb = torch.arange(n, device=dev) * 67 % 251 - 150
+    a = (randn(m * k, 41, dev).view(m, k).double() * 2.0 ** ea.double()[:, None]).float()
+    b = (randn(k * n, 42, dev).view(k, n).double() * 2.0 ** eb.double()[None, :]).float()
+    c = torch.zeros(m * n, device=dev)
+    gk.gemm_unchecked(m, k, n, 1.0, a.view(-1), k, 1, b.reshape(-1), n, 1, 0.0, c, n, 1)
+    got, want = c.view(m, n).double(), a.double() @ b.double()
+    terms = a.abs().double() @ b.abs().double()
+    ok = terms < 2.0 ** 127  # no partial sum overflows
+    # one rounding per k at most, and the subnormal grid
+    bound = (k + 4) * (2.0 ** -24 * terms + 2.0 ** -149)
+    assert ((got - want).abs()[ok] <= bound[ok]).all()
+    assert (terms[ok] < 2.0 ** -126).any() and (terms[ok] > 2.0 ** 110).any()
+
+
+@pytest.mark.parametrize("m,k,n", [(600, 150, 500), (1400, 131, 1300)])
+def test_tiny_values_take_no_second_pass(dev, m, k, n):
+    """Elements far below the others change no output, so none may come from the f32
+    instructions, whose order of sums is another."""
+    a, b = randn(m * k, 51, dev).view(m, k), randn(k * n, 52, dev).view(k, n)
+    tiny = torch.tensor([1e-31, 1e-36, -1e-38, 1e-41, -1e-45], device=dev)
+    out = []
+    for scale in (0.0, 1.0):
+        x, y = a.clone().view(-1), b.clone().view(-1)
+        for t in (x, y):
+            at = torch.arange(0, t.numel(), 997, device=dev)
+            t[at] = scale * tiny[at % 5]
+        c = torch.zeros(m * n, device=dev)
+        gk.gemm_unchecked(m, k, n, 1.0, x, k, 1, y, n, 1, 0.0, c, n, 1)
+        out.append(c)
+    assert torch.equal(out[0], out[1])
 
 
 @pytest.mark.parametrize("specials", [False, True])
