@@ -718,23 +718,30 @@ bool plan_tail_split(int64_t M, int64_t N, int64_t kbytes, EpiKind kind, InType 
 // na < N, tile `tb` over [na, N) at pitch pn_b.
 struct MmaPlan { Tile ta; int32_t pn_a; int64_t na; Tile tb; int32_t pn_b; };
 
-// ld_b: B^T's row stride in bytes.  The wide and strip tiles address 384 and
-// 352 rows of B^T with 32-bit offsets from the panel's first row, so they are
-// taken only when those rows plus the K bytes stay below 2^31 (the 256-row
-// tiles are covered by the stride limit the caller enforces by packing).
 // One round of 128 x 256 tiles on 16x16 MFMAs (T128x256w8m16): products with too
 // few 256 x 256 tiles for the CUs whose half tiles fill at least 9/16 of them in
 // one round.  bf16 2048 x 4096 x 4096 (256 tiles) 58.2 us against 72.7 with the
 // 256 x 128 tiles on 32x32 MFMAs the model picks, 2048 x 2048 x 2304 (144 tiles)
 // 29.6 against 35.2, int8 34.2 against 43.6 and 14.0 against 22.2, K of 256 10.2
 // against 13.0 and 9.5 against 10.1; with 128 tiles (2048^3) half the CUs idle: bf16
-// 28.7 against 22.0.
-bool half16_round(int64_t M, int64_t N, int64_t kbytes, InType in) {
+// 28.7 against 22.0.  Not where 128 x 128 tiles fit one round too, a last column of
+// tiles mostly padding: those are half the work (9300 x 4096 x 257: bf16 38 us against
+// 50, int8 21 against 29, requantized 24 against 32; 10000 x 256 x 300 bf16 7.7 against
+// 9.1), except for i32 output of a short K, which its stores bound (9300 x 512 x 384:
+// 7.5 us against 8.2).  With more padding but two rounds of those the half tile
+// still wins (12288 x 4096 x 300: bf16 51 against 67, requantized 32 against 38;
+// 130 x 4096 x 20000: 51 against 60, 33 against 34).
+bool half16_round(int64_t M, int64_t N, int64_t kbytes, EpiKind kind, InType in) {
     const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
-    const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256);
-    return m16_allowed(in, kbytes) && 16 * tiles >= 9 * cus && tiles <= cus;
+    const int64_t rows = (M + 127) / 128, tiles = rows * ((N + 255) / 256);
+    return m16_allowed(in, kbytes) && 16 * tiles >= 9 * cus && tiles <= cus &&
+           (rows * ((N + 127) / 128) > cus || (kind == EpiKind::I32 && kbytes <= 1024));
 }
 
+// ld_b: B^T's row stride in bytes.  The wide and strip tiles address 384 and
+// 352 rows of B^T with 32-bit offsets from the panel's first row, so they are
+// taken only when those rows plus the K bytes stay below 2^31 (the 256-row
+// tiles are covered by the stride limit the caller enforces by packing).
 bool wide_fits(const TileCand &c, int64_t ld_b, int64_t kbytes) {
     return panels_fit(1, c.bn, 0, ld_b, kbytes);
 }
@@ -765,7 +772,7 @@ MmaPlan plan_mma(int64_t M, int64_t N, int64_t batch, int64_t kbytes, EpiKind ki
         // (a forced wide tile whose rows do not fit is refused at launch)
         return MmaPlan{t, p, N, t, 0};
     }
-    if (batch == 1 && wide_round_enabled() && half16_round(M, N, kbytes, in))
+    if (batch == 1 && wide_round_enabled() && half16_round(M, N, kbytes, kind, in))
         return MmaPlan{Tile::T128x256w8m16, 0, N, Tile::T128x256w8m16, 0};
     MmaPlan plan{t, 0, N, t, 0};
     TailSplit ts;

@@ -93,6 +93,21 @@ def test_wide_round_past_352_takes_the_384_tile(clean_env):
         ("256x384w8k128", 376, 0, "256x384w8k128", 0)
 
 
+@pytest.mark.parametrize("dtype,kind,esz", [("bf16", "bf16", 2), ("i8", "q8", 1), ("i8", "i32", 1)])
+@pytest.mark.parametrize("m,n,half", [
+    (9300, 257, False),   # 73 x 3 tiles of 128 x 128 on 256 CUs
+    (10800, 300, False), (11008, 257, True),  # 85 x 3, 86 x 3
+    (2048, 2304, True), (2048, 4096, True), (130, 20000, True), (12288, 300, True),
+    (2048, 2048, False), (2048, 4097, False),  # 128 and 272 tiles
+])
+def test_half_tile_round(clean_env, dtype, kind, esz, m, n, half):
+    """The 128 x 256 tile takes products of 144 to 256 of them, but not where 128 x 128
+    tiles need no more rounds (i32 output of a short K apart)."""
+    for k in (1024, 4096):
+        short = kind == "i32" and k == 1024 and m > 9000
+        assert (gk.debug_plan(dtype, kind, m, n, k * esz)[0] == "128x256w8m16") == (half or short)
+
+
 def test_no_wide_round_when_256_wide_tiles_fit_one_round(clean_env):
     # 4096^2: 16 x 16 tiles of 256 already make one round
     assert gk.debug_plan("i8", "i32", 4096, 4096, 4096, pitches=True) == \
