@@ -94,6 +94,7 @@ TILE_NAMES = {0: "256x256", 1: "256x128", 2: "128x128", 3: "64x64", 4: "256x256w
               5: "256x128o2", 6: "256x256k128", 7: "256x256w8k128", 8: "128x192k128",
               9: "128x96k128o2", 10: "256x384w8k128",
               11: "256x352w8k128", 12: "256x256w8m16", 13: "256x352w8m16", 14: "128x256w8m16"}
+_PLAN_NAMES = {**TILE_NAMES, 15: "f32x"}
 _IN_CODES = {"i8": 0, "bf16": 1, "f32": 2}
 _KIND_CODES = {"i32": 0, "f32": 1, "bf16": 2, "q8": 3}
 
@@ -105,15 +106,16 @@ def debug_plan(in_type: str, kind: str, m: int, n: int, kbytes: int, batch: int 
     `kbytes` bytes of K per row (and B^T rows `ld_b` bytes apart, 0 for
     packed rows), as (tile, na, tile_b): na > 0 means a second launch covers
     columns [na, n) with tile_b.  pitches=True: (tile, pitch, na, tile_b,
-    pitch_b), a pitch of 0 meaning the tile's width.  Host-only."""
+    pitch_b), a pitch of 0 meaning the tile's width.  "f32x" is the split-bf16
+    kernel, which takes the f32 products of no tile.  Host-only."""
     t, na, tb = C.c_int32(), C.c_int64(), C.c_int32()
     pa, pb = C.c_int32(), C.c_int32()
     _check(_lib.lib().gk_debug_plan(_IN_CODES[in_type], _KIND_CODES[kind], m, n, batch, kbytes,
                                     ld_b, C.byref(t), C.byref(na), C.byref(tb), C.byref(pa),
                                     C.byref(pb)))
     if pitches:
-        return TILE_NAMES[t.value], pa.value, na.value, TILE_NAMES[tb.value], pb.value
-    return TILE_NAMES[t.value], na.value, TILE_NAMES[tb.value]
+        return _PLAN_NAMES[t.value], pa.value, na.value, _PLAN_NAMES[tb.value], pb.value
+    return _PLAN_NAMES[t.value], na.value, _PLAN_NAMES[tb.value]
 
 
 def set_synchronous(on: bool) -> None:

@@ -822,6 +822,31 @@ int choose_splits(int64_t M, int64_t N, int64_t k, size_t esz) {
                                   kMaxSplits);
 }
 
+// Shortest K of the split-bf16 f32 tiles.
+constexpr int64_t kF32xMinK = 128;
+
+// Whether an f32 product runs on the bf16 matrix cores (f32x.hip), given its K
+// ranges on the tiles otherwise: K of 128 or more (below that its four or fewer
+// stages do not pay for its start: 951 x 104 x 2368 with k-contiguous operands 15.7
+// us against 13.9 on the f32 tiles), and no split, or more than one round of the
+// 32 x 32 blocks of small_f32 while its waves' shares are short (two rounds, 1500 x K x
+// 300: 9.6 us against 16.5 at K = 320, 20 against 25 at 1024, 66 against 89 at 4096;
+// K of 385 to 512, one group of loads for each of small_f32's waves, 11.5 to 12.4
+// against 11.7 to 12.6, and with little of the second round, 1200 x 512 x 220, 12.3
+// against 10.6, for two thirds of its error).  A forced tile is
+// taken as asked; GEMMKIT_HIP_F32X=0 turns the route off.
+bool f32x_route(int64_t M, int64_t N, int64_t k, int splits) {
+    const char *s = getenv("GEMMKIT_HIP_F32X");
+    if (s && !strcmp(s, "0")) return false;
+    bool forced;
+    (void)env_tile(&forced);
+    if (forced || k < kF32xMinK || !f32x_fits(M, N)) return false;
+    const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
+    const int64_t blocks = ((M + 31) / 32) * ((N + 31) / 32);
+    return splits == 1 || (small_f32_enabled() && blocks > cus &&
+                           (blocks + cus - 1) / cus * ((k + 31) / 32) <= 256);
+}
+
 // Device memory a call may use for packed operands and split-K partial sums:
 // the workspace arena (grown on demand), or a fixed region handed down (the
 // no-allocation entry point's static scratch, or the inner calls of a K-sliced
@@ -883,8 +908,6 @@ constexpr int64_t kSlabMax = int64_t(64) << 20;
 constexpr int64_t kSliceBytes = int64_t(4) << 20;
 // Longest K the wavefront GEMV takes in one launch.
 constexpr int64_t kGemvMaxK = INT32_MAX;
-// Shortest K of the split-bf16 f32 tiles.
-constexpr int64_t kF32xMinK = 128;
 // Shortest row the unit-row-stride GEMV takes: one 16-byte chunk for each of
 // a workgroup's 64 slots.
 constexpr int64_t kGemvColsMinBytes = 1024;
@@ -1138,11 +1161,9 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     //    CUs) in one launch, a workgroup per 32 x 32 block with K split over its 16
     //    waves, when the blocks fit one round of the CUs (512^3: 7.3 us against 13.8
     //    on f32x, 200 x 150 x 120 5.5 against 7.7) and each wave's share is short;
-    //  * f32x: split into bf16 parts on the bf16 matrix cores, whatever else has K
-    //    of 128 or more (below that its four or fewer stages do not pay for its
-    //    start: 951 x 104 x 2368 with k-contiguous operands 15.7 us against 13.9 on
-    //    the f32 tiles; 1500 x 130 x 1500 14.3 against 25.1; 2048^3: 88 us against 140 on the f32 tiles;
-    //    1536 x 640 x 167, two rounds of blocks: 15 us against 24 with small_f32).
+    //  * f32x: split into bf16 parts on the bf16 matrix cores (1500 x 130 x 1500 15.7
+    //    us against 24.7 on the f32 tiles; 2048^3: 109 against 138; 1536 x 167 x 640,
+    //    two rounds of blocks: 8 against 16 with small_f32).
     if (in == InType::F32 && !vector_route) {
         const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
         const int64_t blocks = ((M + 31) / 32) * ((N + 31) / 32);
@@ -1154,9 +1175,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
             if (e != hipSuccess) return hip_fail(e, "small f32 gemm launch");
             return finish("small f32 gemm");
         }
-        if (k >= kF32xMinK && f32x_fits(M, N) &&
-            (splits == 1 || (small_f32_enabled() && blocks > cus &&
-                             (blocks + cus - 1) / cus * ((k + 31) / 32) <= 256))) {
+        if (f32x_route(M, N, k, splits)) {
             // Every tile row or column reads an operand again, a cache line for a few
             // elements where neither of its strides is short: such an operand is packed
             // first (the sums do not depend on it).  2048^3 with every second column of
@@ -2136,6 +2155,14 @@ int gk_debug_plan(int32_t in, int32_t kind, int64_t m, int64_t n, int64_t batch,
         kbytes < 0 || ld_b < 0 || !tile || !na || !tile_b)
         return fail(GK_ERR_ARG, "gemmkit: gk_debug_plan: bad argument");
     if (ld_b == 0) ld_b = (kbytes + 15) / 16 * 16;
+    if (in == 2 && std::min(m, n) > 16 &&
+        f32x_route(m, n, kbytes / 4, choose_splits(m, n, kbytes / 4, 4))) {
+        *tile = *tile_b = (int32_t)Tile::F32x;
+        *na = 0;
+        if (pn_a) *pn_a = 0;
+        if (pn_b) *pn_b = 0;
+        return ok();
+    }
     const MmaPlan plan = plan_mma(m, n, batch, kbytes, (EpiKind)kind, (InType)in, ld_b);
     *tile = (int32_t)plan.ta;
     *na = plan.na < n ? plan.na : 0;

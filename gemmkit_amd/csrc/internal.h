@@ -103,6 +103,7 @@ enum class Tile : int {
     T256x352w8k128 = 11,  // likewise, 2 x 4 waves over 256 x 256 plus a 96-column strip
     T256x256w8m16 = 12,  // 8 waves, 128-byte stages, 2-stage ring, 16x16 MFMAs (mma16.hip)
     T128x256w8m16 = 14,  // T256x256w8m16 on half the rows (mma16.hip)
+    F32x = 15,           // no tile of launch_mma: the split-bf16 f32 kernel (f32x.hip), in plans only
     T256x352w8m16 = 13,  // 8 waves (4 x 2), 16x16 MFMAs, ping-pong, one round at a column pitch (mma16w.hip)
 };
 

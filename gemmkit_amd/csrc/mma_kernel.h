@@ -985,6 +985,7 @@ static hipError_t launch_tile(Tile tile, const MmaArgs &args, const EpiParams &e
     case Tile::T256x256w8m16: break;  // mma16.hip (launch_mma dispatches it first)
     case Tile::T256x352w8m16: break;  // mma16w.hip (likewise)
     case Tile::T128x256w8m16: break;  // mma16.hip
+    case Tile::F32x: break;           // f32x.hip (launched as such)
     }
     return hipErrorInvalidValue;
 }

@@ -55,7 +55,8 @@ const char *gk_version(void);
  * output, K bytes per operand row; in: 0 int8, 1 bf16, 2 f32; kind: 0 i32,
  * 1 f32, 2 bf16, 3 requantized i8/u8 output; ld_b: B^T's row stride in bytes,
  * 0 for rows of K bytes rounded up to 16), as the dispatcher would choose
- * it with the current environment: *tile is the tile of the (first) launch,
+ * it with the current environment: *tile is the tile of the (first) launch (15
+ * for f32 products on the split-bf16 kernel),
  * *na the kernel-frame columns it covers when the product is split into two
  * launches (else 0), *tile_b the tile of the second launch, *pn_a and *pn_b
  * (either may be NULL) the two launches' column pitches (0: the tile's

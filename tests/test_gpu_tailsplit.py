@@ -153,7 +153,8 @@ def test_bf16_fused_bias_relu(dev):
     assert ((got - ref).abs() <= 1e-2 * torch.maximum(ref.abs(), floor)).all()
 
 
-def test_f32(dev):
+def test_f32(dev, monkeypatch):
+    monkeypatch.setenv("GEMMKIT_HIP_F32X", "0")  # the f32 tiles
     m, k, n = 2048, 2048, 8448
     plans(("f32", "f32", m, n, 4 * k), wide=False)  # f32 inputs never take the wide plan
     g = torch.Generator().manual_seed(8)

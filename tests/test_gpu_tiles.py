@@ -88,8 +88,8 @@ def test_float_tiles_identical(dev, dt):
     c0 = torch.randn(m * n, generator=g).to(dev)
     outs = {}
     for name in TILES_F:
-        if name == M16 and dt == torch.float32:
-            continue
+        if name in (M16, "128x256w8m16") and dt == torch.float32:
+            continue  # no f32 kernels
         c = c0.clone()
         with tile(name):
             if dt == torch.bfloat16:
@@ -99,7 +99,7 @@ def test_float_tiles_identical(dev, dt):
                 gk.gemm(0.5, gk.MatRef.from_row_major(a, m, k), gk.MatRef(b, k, n, 1, k), 1.0,
                         gk.MatMut.from_row_major(c, m, n))
         outs[name] = c
-    same = [t for t in TILES_F if t != M16]
+    same = [t for t in TILES_F if t in outs and t != M16]
     first = outs[same[0]]
     for name in same[1:]:
         assert torch.equal(outs[name], first), name
@@ -108,6 +108,33 @@ def test_float_tiles_identical(dev, dt):
     for name in [same[0]] + ([M16] if M16 in outs else []):
         err = (outs[name].double().cpu().reshape(m, n) - ref).norm() / ref.norm()
         assert err <= (1e-5 if dt == torch.float32 else 1e-2), name
+
+
+def test_forced_f32_tile_is_taken(dev):
+    """A forced tile runs also where f32 products take the split-bf16 kernel by
+    themselves: one sum per element, rounded along K, against several (and with the
+    kernel switched off the tiles' bits by themselves)."""
+    m, k, n = 900, 272, 1000
+    g = torch.Generator().manual_seed(22)
+    a, b = torch.randn(m * k, generator=g).to(dev), torch.randn(k * n, generator=g).to(dev)
+
+    def call():
+        c = torch.zeros(m * n, device=dev)
+        gk.gemm(1.0, gk.MatRef.from_row_major(a, m, k), gk.MatRef(b, k, n, 1, k), 0.0,
+                gk.MatMut.from_row_major(c, m, n))
+        return c
+
+    own = call()
+    with tile("128x128"):
+        forced = call()
+    os.environ["GEMMKIT_HIP_F32X"] = "0"
+    try:
+        tiles = call()
+    finally:
+        del os.environ["GEMMKIT_HIP_F32X"]
+    assert torch.equal(forced, tiles) and not torch.equal(forced, own)
+    with tile(M16), pytest.raises(gk.GemmkitError):  # no f32 kernel of that tile
+        call()
 
 
 @pytest.mark.parametrize("name", TILES_F)

@@ -39,6 +39,7 @@ def clean_env(monkeypatch):
     monkeypatch.delenv("GEMMKIT_HIP_TAILSPLIT", raising=False)
     monkeypatch.delenv("GEMMKIT_HIP_WIDE", raising=False)
     monkeypatch.delenv("GEMMKIT_HIP_M16", raising=False)
+    monkeypatch.delenv("GEMMKIT_HIP_F32X", raising=False)
 
 
 @pytest.fixture
@@ -52,12 +53,30 @@ def pick_only(no_wide, monkeypatch):
 
 
 @pytest.mark.parametrize("shape,best", SWEEP)
-def test_model_picks_the_measured_best_tile(pick_only, shape, best):
+def test_model_picks_the_measured_best_tile(pick_only, monkeypatch, shape, best):
+    monkeypatch.setenv("GEMMKIT_HIP_F32X", "0")  # f32: the tiles' own choice
     assert gk.debug_plan(*shape)[0] == best
 
 
+def test_f32_products_off_the_tiles(clean_env, monkeypatch):
+    # K of 128 or more on the split-bf16 kernel, also where the tiles would split K
+    # in two rounds of the small kernel's blocks (1500 x 200: 47 x 7)
+    for m, n, k, f32x in ((2048, 2048, 2048, True), (1024, 1024, 128, True),
+                          (1024, 1024, 127, False), (1500, 200, 256, True),
+                          (512, 512, 512, False), (300, 200, 16384, False)):
+        assert (gk.debug_plan("f32", "f32", m, n, 4 * k)[0] == "f32x") == f32x, (m, n, k)
+    assert gk.debug_plan("bf16", "f32", 2048, 2048, 4096)[0] != "f32x"
+    assert gk.debug_plan("f32", "f32", 2048, 2048, 8192, pitches=True) == ("f32x", 0, 0, "f32x", 0)
+    monkeypatch.setenv("GEMMKIT_HIP_F32X", "0")
+    assert gk.debug_plan("f32", "f32", 2048, 2048, 8192)[0] == "128x128"
+    monkeypatch.delenv("GEMMKIT_HIP_F32X")
+    monkeypatch.setenv("GEMMKIT_HIP_TILE", "64x64")
+    assert gk.debug_plan("f32", "f32", 2048, 2048, 8192)[0] == "64x64"
+
+
 def test_m16_tile_exclusions(pick_only, monkeypatch):
-    # no f32 variant of the 16x16-MFMA tile
+    # no f32 variant of the 16x16-MFMA tile (with f32 products on the tiles at all)
+    monkeypatch.setenv("GEMMKIT_HIP_F32X", "0")
     assert gk.debug_plan("f32", "f32", 4096, 4096, 16384)[0] != "256x256w8m16"
     # bf16 contractions of at most 256 bytes stay on the 32x32 tiles (the
     # streaming kernel's summation order); int8 sums are exact either way
@@ -108,13 +127,14 @@ def test_half_tile_round(clean_env, dtype, kind, esz, m, n, half):
         assert (gk.debug_plan(dtype, kind, m, n, k * esz)[0] == "128x256w8m16") == (half or short)
 
 
-def test_no_wide_round_when_256_wide_tiles_fit_one_round(clean_env):
+def test_no_wide_round_when_256_wide_tiles_fit_one_round(clean_env, monkeypatch):
     # 4096^2: 16 x 16 tiles of 256 already make one round
     assert gk.debug_plan("i8", "i32", 4096, 4096, 4096, pitches=True) == \
         ("256x256w8m16", 0, 0, "256x256w8m16", 0)
     # batched products never take it (per element shape only), nor f32
     # inputs (2048 x 11008 x 4096: 1379 against 1328 us)
     assert gk.debug_plan("i8", "q8", 2048, 11008, 4096, 2)[0] != "256x384w8k128"
+    monkeypatch.setenv("GEMMKIT_HIP_F32X", "0")
     assert gk.debug_plan("f32", "f32", 2048, 11008, 16384)[0] != "256x384w8k128"
 
 
