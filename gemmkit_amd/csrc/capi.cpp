@@ -914,6 +914,32 @@ constexpr int64_t kGemvColsMinBytes = 1024;
 // ... and most rows (a grid of at most 2^32 threads).
 constexpr int64_t kColsMaxRows = 1 << 26;
 
+// Whether a batch of vector products that share one R x K matrix of unit row stride
+// packs it: one pack serves the batch, and the row kernels read a short k-contiguous
+// row faster than the in-place ones its columns (which read 128 bytes at a time and
+// end in an exchange or a second launch).  Both sides measured over K 256 to 4096, R 64
+// to 4096 and up to 2048 elements; time in place over time packed:
+//   f32, K of 512 or less           1.03 to 2.5   (1 x 256 x 1024 times 256: 40 us, 21)
+//   one vector, K of 2048 bytes     1.02 to 1.6   (bf16 1 x 1024 x 1024: 46, 39)
+//   one vector, a matrix of 1 to 2 MB in a long batch (bf16 1 x 2048 x 512 times 2048:
+//   276, 212), other matrices       0.5 to 0.9
+//   bf16 5 to 16 vectors, short K   1.0 to 1.4    (8 x 512 x 512 times 4096: 530, 375)
+// and below these lines 0.3 to 1.0; small batches gain too little to pay for the pack.
+bool shared_packs(InType in, int64_t nvec, int64_t R, int64_t kbytes, int64_t batch) {
+    const int64_t outs = batch * R * nvec;
+    const bool bf16 = in == InType::BF16;
+    if (in == InType::I8) return false;
+    if (nvec == 1 || !bf16)
+        return (kbytes <= 2048 && outs >= 1 << 17) ||
+               (nvec == 1 && kbytes <= 4096 && outs >= 1 << 19 &&
+                R * kbytes <= (bf16 ? 8 : 5) << 18);
+    if (nvec <= 4) return false;
+    if (nvec <= 8)
+        return (kbytes <= 1280 && outs >= 1 << 20) ||
+               (kbytes <= 3072 && outs >= 4 << 20 && R * kbytes <= 1 << 20);
+    return kbytes <= 1792 && outs >= 3 << 17;
+}
+
 int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int64_t n,
             const void *a, int64_t rsa, int64_t csa, int64_t bsa, const void *b, int64_t rsb,
             int64_t csb, int64_t bsb, void *c, int64_t rsc, int64_t csc, int64_t bsc,
@@ -1099,12 +1125,12 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // x 4096: 11.5 against 18.9), and reads a row-major matrix in place in any case.
     const Opnd &mat_op = vec_is_a ? Bt : A;
     const int64_t long_side = std::max(M, N);
-    const bool mat_cols = mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
-                          long_side <= kColsMaxRows;
+    const bool unit_rows = mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
+                           long_side <= kColsMaxRows;
     const bool long_vec = skinny_is_long(in, k, (int)std::min<int64_t>(short_side, 16));
     const bool long_ok =
         short_side <= 8 ? short_side > (in == InType::BF16 ? 2 : kGemvColsMaxVec)
-                        : (in == InType::I8 && mat_cols) ||
+                        : (in == InType::I8 && unit_rows) ||
                               (long_side >= 16 * (int64_t)(g_num_cus > 0 ? g_num_cus : 256) &&
                                (in != InType::BF16 || kbytes <= 16384));
     const bool skinny_ok = short_side >= 2 && short_side <= 16 && !gemv_first &&
@@ -1115,6 +1141,15 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
                       (vec_is_a ? a_ok : b_ok) &&
                       skinny_lds_bytes(in, k, (int)short_side) > 80 * 1024));
     const bool vector_route = skinny_ok || short_side <= 8;
+    const bool vec_in_place = skinny_ok && !skinny_long;  // staged from any strides
+    const bool shared = unit_rows && batch > 1 && mat_op.bs == 0 &&
+                        shared_packs(in, short_side, long_side, kbytes, batch) &&
+                        region_fits(rg, pack_bytes(in, long_side, k, batch, mat_op) +
+                                            (vec_in_place || (vec_is_a ? a_ok : b_ok)
+                                                 ? 0
+                                                 : pack_bytes(in, short_side, k, batch,
+                                                              vec_is_a ? A : Bt)));
+    const bool mat_cols = unit_rows && !shared;
     // A GEMV whose matrix has unit row stride (x * W with W row-major) reads
     // both operands in place instead of packing the matrix first, three
     // passes over it (bf16 1 x 4096 x 11008: 17 against 55 us), once K is long
@@ -1138,7 +1173,6 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
                            (rounds <= 16 || long_side * kbytes >= rounds * (3 << 18));
     const bool cols = gemv_cols || skinny_cols;
     const bool cols_pack_vec = cols && (vec_is_a ? A : Bt).ks != 1;
-    const bool vec_in_place = skinny_ok && !skinny_long;  // staged from any strides
     const bool pack_a = cols ? vec_is_a && cols_pack_vec : !a_ok && !(vec_in_place && vec_is_a);
     const bool pack_b = cols ? !vec_is_a && cols_pack_vec : !b_ok && !(vec_in_place && !vec_is_a);
     // Split K.  Float products split by the element shape only (a batched
@@ -1221,15 +1255,23 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     const int64_t kchunk = splits > 1 ? round_up64((k + splits - 1) / splits, 64 / (int64_t)esz) : k;
     // Batch elements per split-K launch: as many as kSlabMax of partial sums
     // holds (at least one).
-    const int64_t elem_part = (int64_t)splits * M * N * 4;
-    const int64_t zchunk = splits > 1 ? std::max<int64_t>(1, std::min(batch, kSlabMax / elem_part)) : batch;
+    // (skinny_cols: a batch may share its matrix, so the partial sums are bounded too;
+    // twice the bytes, since a chunk of 64 MiB costs 5% in its two launches: bf16 2048 x
+    // (4 x 512 x 300) 133 us against 127)
+    auto skinny_part = [&](int64_t nb) {
+        return skinny_cols_part_bytes(in, long_side, k, (int)short_side, nb, g_num_cus);
+    };
+    const int64_t elem_part = splits > 1 ? (int64_t)splits * M * N * 4
+                              : skinny_cols ? skinny_part(1) : 0;
+    const int64_t zchunk =
+        elem_part ? std::max<int64_t>(1, std::min(batch, (splits > 1 ? 1 : 2) * kSlabMax / elem_part))
+                  : batch;
     const size_t part_bytes =
         splits > 1 ? (size_t)round_up64(zchunk * elem_part, 256)
         : gemv_cols
-            ? (size_t)gemv_cols_part_bytes(in, std::max(M, N), k, (int)short_side, batch, g_num_cus)
-        : skinny_cols
-            ? (size_t)skinny_cols_part_bytes(in, std::max(M, N), k, (int)short_side, batch, g_num_cus)
-            : 0;
+            ? (size_t)gemv_cols_part_bytes(in, long_side, k, (int)short_side, batch, g_num_cus)
+        : skinny_cols ? (size_t)std::max(skinny_part(zchunk), skinny_part((batch - 1) % zchunk + 1))
+                      : 0;
 
     uint8_t *part = nullptr;
     if (pack_a || pack_b || part_bytes) {
@@ -1270,8 +1312,20 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         g.K = (int32_t)k;
         g.cus = g_num_cus;
         g.batch = (int32_t)batch;
-        e = skinny_cols ? launch_skinny_cols(in, g, eg, tl_stream)
-            : skinny_long ? launch_skinny_long(in, g, eg, tl_stream)
+        if (skinny_cols) {
+            for (int64_t z0 = 0; z0 < batch; z0 += zchunk) {
+                GemvArgs gz = g;
+                gz.batch = (int32_t)std::min(zchunk, batch - z0);
+                gz.mat = ptr_add(g.mat, z0 * g.bsm * (int64_t)esz);
+                gz.vec = ptr_add(g.vec, z0 * g.bsv * (int64_t)esz);
+                EpiParams ez = eg;
+                ez.c = (void *)ptr_add(eg.c, z0 * bsc * out_size(ep.kind));
+                e = launch_skinny_cols(in, gz, ez, tl_stream);
+                if (e != hipSuccess) return hip_fail(e, "skinny launch");
+            }
+            return finish("skinny");
+        }
+        e = skinny_long ? launch_skinny_long(in, g, eg, tl_stream)
             : skinny_ok ? launch_skinny(in, g, eg, tl_stream)
             : gemv_cols ? launch_gemv_cols(in, g, eg, tl_stream)
                         : launch_gemv(in, g, eg, tl_stream);

@@ -84,6 +84,75 @@ def test_batch_and_packed_equal_standalone(dev, dtype):
         assert torch.equal(pk.view(n, m).T.reshape(-1), one)
 
 
+def shared_batch(dev, dtype, batch, m, k, n, ws):
+    """A batch on one row-major matrix (zero batch stride), strided in C."""
+    dt = DT[dtype]
+    a, b = values(batch * m * k, dt, 7, dev), values(k * n, dt, 8, dev)
+    cbs = m * n + 5
+    c = torch.zeros(batch * cbs, dtype=dt, device=dev)
+
+    def call(ws=ws):
+        gk.gemm_batched_unchecked(batch, m, k, n, 1.0, a, k, 1, m * k, b, n, 1, 0, 0.0, c, n, 1,
+                                  cbs, ws=ws)
+
+    def check():
+        for z in (0, 1, batch // 2, batch - 2, batch - 1):
+            one = torch.zeros(m * n, dtype=dt, device=dev)
+            gk.gemm_unchecked(m, k, n, 1.0, a, k, 1, b, n, 1, 0.0, one, n, 1, a_off=z * m * k)
+            assert torch.equal(c[z * cbs:z * cbs + m * n], one), z
+        assert (c.view(batch, cbs)[:, m * n:] == 0).all()
+
+    return call, check, c
+
+
+@pytest.mark.parametrize("dtype,batch,m,k,n", [("bf16", 1500, 8, 1100, 600),
+                                               ("f32", 1000, 16, 1000, 520),
+                                               ("bf16", 400, 8, 8200, 1000)])
+def test_shared_matrix_bounded_workspace(dev, dtype, batch, m, k, n):
+    """Each element's partial sums (16 f32 slabs of its output beyond the LDS, 8
+    below) would take 205 to 266 MB at once: at most 128 MiB are used at a time."""
+    ws = gk.Workspace()
+    call, check, _ = shared_batch(dev, dtype, batch, m, k, n, ws)
+    call()
+    assert (16 if k > 8192 else 8) * batch * m * n * 4 > 200e6
+    assert ws.bytes() <= 130 << 20
+    check()
+
+
+@pytest.mark.parametrize("dtype,batch,m,k,n", [
+    ("f32", 300, 1, 256, 500), ("f32", 150, 3, 500, 333), ("f32", 40, 9, 300, 400),
+    ("bf16", 300, 1, 700, 500), ("bf16", 600, 7, 600, 260), ("bf16", 100, 13, 800, 400)])
+def test_shared_matrix_of_short_rows_is_packed(dev, dtype, batch, m, k, n):
+    """One pack serves the batch; under capture, where the workspace cannot grow, one
+    vector's matrix is read in place: the same bits every way."""
+    ws = gk.Workspace()
+    call, check, c = shared_batch(dev, dtype, batch, m, k, n, ws)
+    call()
+    pad = 16 // DT[dtype].itemsize
+    assert ws.bytes() >= n * (k + pad - 1) // pad * pad * DT[dtype].itemsize
+    assert ws.bytes() < 8 * batch * m * n * 4 or m == 1
+    check()
+    # captured: with the arena of that call, and one vector with none
+    for arena in (ws, gk.Workspace()):
+        if arena is not ws and m > 1:  # (more vectors have partial sums in the workspace)
+            continue
+        held = arena.bytes()
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        gk.set_synchronous(False)
+        try:
+            with torch.cuda.graph(graph):
+                call(arena)
+        finally:
+            gk.set_synchronous(True)
+        assert arena.bytes() == held
+        for _ in range(3):
+            c.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            check()
+
+
 def test_nonfinite_columns_stay_apart(dev):
     """A row of infinities or NaN reaches its own outputs only, past K neither."""
     m, k, n = 3, 1030, 50
