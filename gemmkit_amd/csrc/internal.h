@@ -211,7 +211,7 @@ struct PackJob {
     void *dst;
     int64_t ld;
     int32_t batch;
-    int32_t blocks, copy, p0, p1;  // set by launch_pack
+    int32_t blocks, copy, p0, p1;  // set by launch_pack (copy: chunks per workgroup, 0: transposed)
 };
 // One or two packs, in one launch where their strides allow it.
 hipError_t launch_pack(InType in, PackJob *jobs, int n, hipStream_t stream);

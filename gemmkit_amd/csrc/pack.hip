@@ -129,8 +129,12 @@ __device__ __forceinline__ v4u_p shift_down(v4u_p v, int sh) {
 // k-contiguous rows (element (r, p) at r*rs + p) whose base, stride or length
 // misses the 16-byte alignment: a copy of 16 bytes per lane.  Bound by memory,
 // by latency below a few MB.  2^llog lanes (at most 64) walk a row's chunks, a
-// lane takes four rows at a time, and a workgroup at most kCopyChunks chunks of
-// its rows.  A row's last chunk is the 16 bytes before the row's end, shifted
+// lane takes four rows at a time, and a workgroup at most j.copy chunks of its
+// rows: kCopyChunks, or one per lane while that leaves fewer workgroups than CUs
+// (a lane's chunks are round trips in series: i8 32 x 4665 times 4665 x 2 in all 11.6
+// us with two workgroups, 9.6 with ten, as through pack_kernel; with a k-contiguous
+// right side 8.2, 6.2 and 9.3).
+// A row's last chunk is the 16 bytes before the row's end, shifted
 // down (the caller ensures K >= EPV), so no lane goes element by element.
 // i8 777 x 1001: 3.8 us against 4.6 through pack_kernel, 11008 x 4097: 22 against 38.
 constexpr int kCopyChunks = 256, kCopyRows = 4;
@@ -143,8 +147,8 @@ __device__ __forceinline__ void pack_copy(const PackJob &j, int block) {
     const int blocks_c = j.p0, llog = j.p1;
     const int lanes = 1 << llog, groups = 256 >> llog;
     const int64_t cpr = ld / EPV;
-    const int64_t c0 = (int64_t)(block % blocks_c) * kCopyChunks;
-    const int64_t c1 = c0 + kCopyChunks < cpr ? c0 + kCopyChunks : cpr;
+    const int64_t c0 = (int64_t)(block % blocks_c) * j.copy;
+    const int64_t c1 = c0 + j.copy < cpr ? c0 + j.copy : cpr;
     const int64_t r0 = (int64_t)(block / blocks_c) * groups * kCopyRows +
                        ((int)threadIdx.x >> llog);
     for (int64_t c = c0 + ((int)threadIdx.x & (lanes - 1)); c < c1; c += lanes) {
@@ -228,9 +232,14 @@ static bool plan_pack(PackJob &j, int64_t epv) {
         int llog = 0;
         while (llog < 6 && (1 << llog) < cpr) ++llog;
         const int64_t rpb = (int64_t)(256 >> llog) * kCopyRows;
-        const int64_t bc = (cpr + kCopyChunks - 1) / kCopyChunks;
-        blocks = bc * ((j.rows + rpb - 1) / rpb);
-        j.copy = 1;
+        const int64_t br = (j.rows + rpb - 1) / rpb;
+        int64_t bc = (cpr + kCopyChunks - 1) / kCopyChunks;
+        j.copy = kCopyChunks;
+        if (bc * br * j.batch < 256) {
+            j.copy = 64;
+            bc = (cpr + 63) / 64;
+        }
+        blocks = bc * br;
         j.p0 = (int)bc;
         j.p1 = llog;
     } else if (j.rs == 1 && j.rows >= epv) {

@@ -32,9 +32,10 @@ def run(batch, m, k, n, a, ra, b, rb, dtype, dev):
 
 # rows x K around the packs' blocks (4, 8 or 16 rows x k per lane, 64..256 per
 # workgroup), row lengths and steps that miss every alignment, and the copy's
-# 1024-chunk workgroups (one row longer than that, many short rows)
+# workgroups: 64 chunks of a few rows (below, at and above one such), 256 of many
+# rows, and many short rows
 SHAPES = [(20, 17, 19), (33, 64, 65), (64, 129, 257), (130, 255, 128), (257, 300, 77),
-          (40, 9001, 35), (300, 24, 1000)]
+          (40, 9001, 35), (300, 24, 1000), (18, 1025, 20), (5000, 4103, 17)]
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "i8"])
