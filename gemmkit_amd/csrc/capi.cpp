@@ -1161,11 +1161,25 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // The skinny kernel likewise, with its sums added in a second launch (bf16
     // 8 x 4096 x 4096: 10.6 us against 25.1; 16 x 1024 x 1024: 5.3 against 8.8); i8
     // sums have no order, so it takes long K from the GEMV there (1 x 16384 x 1024:
-    // two vectors on it 9.9 us, one on the GEMV 16.2).
+    // two vectors on it 9.9 us, one on the GEMV 16.2), and narrow matrices, which
+    // leave the GEMV few workgroups (packed first, GEMV, skinny: 1 x 2048 x 179 6.6,
+    // 10.0, 5.1 us; 2 x 7552 x 64 7.2, 11.1, 5.7; 2 x 4096 x 4096 21.7, 11.3, 8.3; 1 x
+    // 4096 x 4096 21.1, 9.3, 8.0 but 1 x 2528 x 4096 16.6, 8.4, 9.7 and 2 x 4096 x 8000
+    // 34, 12.9, 14.4) while its partial sums have room.
+    const bool i8_narrow =
+        short_side == 2 ? long_side <= 4096
+                        : short_side == 1 && (long_side <= 512 ||
+                                              (long_side <= 1024 && (k < 2048 || k % 128 == 0)));
+    const Opnd &vec_op = vec_is_a ? A : Bt;
     const bool skinny_cols =
         mat_cols && long_side >= kSkinnyColsMinRows &&
-        (skinny_ok || (in == InType::I8 && short_side <= kGemvColsMaxVec && k > 8192 && k_fits &&
-                       skinny_enabled()));
+        (skinny_ok ||
+         (in == InType::I8 && short_side <= kGemvColsMaxVec && k_fits && skinny_enabled() &&
+          (k > 8192 ||
+           (i8_narrow &&
+            region_fits(rg, (size_t)skinny_cols_part_bytes(in, long_side, k, (int)short_side, batch,
+                                                           g_num_cus) +
+                                (vec_op.ks != 1 ? pack_bytes(in, short_side, k, batch, vec_op) : 0))))));
     const int64_t rounds = gemv_cols_rounds(in, k, (int)short_side);
     const bool gemv_cols = vector_route && !skinny_ok && !skinny_cols &&
                            short_side <= kGemvColsMaxVec && mat_cols &&

@@ -20,15 +20,20 @@ def values(n, dt, seed, dev):
     return torch.randn(n, generator=g).to(dt).to(dev)
 
 
+# by default most products of two to four vectors, and narrow i8 ones, take the
+# skinny kernels: "0" keeps all on the GEMV
+@pytest.mark.parametrize("skinny", ["1", "0"])
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "i8"])
 # (vectors, k, n): one batch of chunks per slot and several, K ending inside a
 # chunk, fewer columns than a lane's 16 bytes would leave whole, one group and
 # enough groups to run whole, 256 lanes per row (K rows beyond 8 KiB)
 @pytest.mark.parametrize("shape", [(1, 1024, 16), (1, 1025, 17), (1, 2048, 9000), (1, 4097, 65),
                                    (1, 9001, 33), (1, 16384, 129), (2, 2049, 40), (2, 8200, 100),
-                                   (3, 1500, 130), (4, 2048, 2000), (4, 1031, 31)],
+                                   (3, 1500, 130), (4, 2048, 2000), (4, 1031, 31),
+                                   (1, 2064, 1100), (2, 2500, 4200)],
                          ids=lambda s: "x".join(map(str, s)))
-def test_unit_row_stride_equals_k_contiguous(dev, dtype, shape):
+def test_unit_row_stride_equals_k_contiguous(dev, monkeypatch, dtype, shape, skinny):
+    monkeypatch.setenv("GEMMKIT_HIP_SKINNY", skinny)
     m, k, n = shape
     dt = DT[dtype]
     pad = 16 // dt.itemsize

@@ -29,6 +29,11 @@ def values(n, dt, seed, dev):
                                    # vectors beyond the LDS: one row group, 8-, 16- and
                                    # 32-row ones, K ending inside a step and a chunk,
                                    # more than eight vectors
+                                   # i8: both sides of the widths it takes from the
+                                   # GEMV (512, 1024, 4096 columns)
+                                   (1, 2528, 512), (1, 2528, 513), (1, 2048, 1024),
+                                   (1, 1627, 1025), (2, 2528, 4096), (2, 7552, 4097),
+                                   (1, 1030, 8), (2, 2048, 9),
                                    (8, 16385, 40), (5, 14008, 2049), (8, 8190, 4100),
                                    (7, 9300, 8200), (16, 4104, 2048), (12, 5503, 2100)],
                          ids=lambda s: "x".join(map(str, s)))
