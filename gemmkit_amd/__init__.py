@@ -249,7 +249,7 @@ class MatMut(MatRef):
 def _bf16_bits(x: float) -> int:
     """f32 -> bf16 bit pattern, round to nearest even (NaN quieted).  In integers:
     through a tensor it took 3.8 us, twice per bfloat16 call."""
-    bits = int.from_bytes(C.c_float(float(x)), "little")
+    bits = int.from_bytes(C.c_float(x), "little")  # (numbers only: float() takes text)
     if bits & 0x7FFFFFFF > 0x7F800000:
         return 0xFFFF
     return (bits + 0x7FFF + ((bits >> 16) & 1)) >> 16

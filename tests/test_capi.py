@@ -276,6 +276,13 @@ def test_batched_ptr_empty_is_a_no_op():
     assert _lib.lib().gk_gemm_batched_slice_bf16(None, None, 0, 1) == 0
 
 
+@pytest.mark.parametrize("bad", ["1.0", b"1", None, [1.0], 1j])
+def test_bf16_scalars_are_numbers(bad):
+    import gemmkit_amd as gk
+    with pytest.raises((TypeError, ValueError)):
+        gk._bf16_bits(bad)
+
+
 def test_bf16_scalar_bits_match_torch():
     """alpha, beta and slopes reach the bf16 entries as bits: torch's conversion."""
     import random
@@ -286,6 +293,8 @@ def test_bf16_scalar_bits_match_torch():
     vals = [0.0, -0.0, 1.0, -1.25, 1, True, float("inf"), float("-inf"), float("nan"), 1e40, -1e40,
             3.4028234e38, 3.39e38, 1e-40, 1e-45, 2.0 ** -133, 1.00390625, 1.01171875, -0.99609375]
     vals += [struct.unpack("<f", struct.pack("<I", r.getrandbits(32)))[0] for _ in range(4000)]
+    import numpy as np
+    vals += [np.float32(1.0039), np.float64(-3.3), np.int64(7), torch.tensor(2.7), torch.tensor([0.3])]
     for v in vals:
         want = int(torch.tensor([v], dtype=torch.float32).to(torch.bfloat16).view(torch.int16)
                    .item()) & 0xFFFF
