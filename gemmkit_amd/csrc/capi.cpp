@@ -1115,24 +1115,30 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     const bool vec_is_a = M <= N;
     const bool gemv_first = gemv_beats_skinny(in, short_side, kbytes);
     // Vectors beyond the LDS of a workgroup: 5..8 (bf16 3..8) on skinny_long, fewer on
-    // the GEMV (f32 4 x 16384 x 600: 20 us against 26; bf16 14.3 against 13.0); more of them, whose L2 reads are as large as the matrix's
-    // in 16-row items and twice that in 8-row ones, where 16-row items fill the CUs
-    // and, for bf16, rows are at most 16 KiB: 16 x 4096 x 4096 10.0 us against 12.7
-    // on the split matrix-core tiles, f32 18.1 against 42, i8 16 x 11008 x 4096 13.4
-    // against 14.3; bf16 16 x 11008 x 4096 22.9 against 20.4 and f32 16 x 16384 x
-    // 2500 75 against 51 stay there.  i8, whose sums have no order, takes it with
+    // the GEMV (f32 4 x 16384 x 600: 20 us against 26; bf16 14.3 against 13.0); more of
+    // them, whose L2 reads are as large as the matrix's in 16-row items and twice that
+    // in 8-row ones, where 16-row items fill the CUs and, for bf16, rows are at most 16
+    // KiB: 16 x 4096 x 4096 10.0 us against 12.7 on the split matrix-core tiles, f32
+    // 18.1 against 42, i8 16 x 11008 x 4096 13.4 against 14.3; bf16 16 x 11008 x 4096
+    // 22.9 against 20.4 and f32 16 x 16384 x 2500 75 against 51 stay there.  Between one
+    // and two rounds of 16-row items it gains little or loses to them (bf16 16 x 8000:
+    // 4500 rows 19.9 us against 17.0, 5810 21.0 against 20.1, 7000 24.7 against 22.8, i8
+    // 16 x 16384 alike): a k-contiguous i8 matrix, whose sums have no order, stays on
+    // the tiles there; float ones must sum alike whatever their strides, and a row-major
+    // matrix, read in place, gains far more.  i8 takes skinny_long with
     // 5..8 vectors already where the LDS would hold one workgroup a CU (8 x 11008
     // x 4096: 11.5 against 18.9), and reads a row-major matrix in place in any case.
     const Opnd &mat_op = vec_is_a ? Bt : A;
-    const int64_t long_side = std::max(M, N);
+    const int64_t long_side = std::max(M, N), cus = g_num_cus > 0 ? g_num_cus : 256;
     const bool unit_rows = mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
                            long_side <= kColsMaxRows;
     const bool long_vec = skinny_is_long(in, k, (int)std::min<int64_t>(short_side, 16));
     const bool long_ok =
         short_side <= 8 ? short_side > (in == InType::BF16 ? 2 : kGemvColsMaxVec)
                         : (in == InType::I8 && unit_rows) ||
-                              (long_side >= 16 * (int64_t)(g_num_cus > 0 ? g_num_cus : 256) &&
-                               (in != InType::BF16 || kbytes <= 16384));
+                              (long_side >= 16 * cus &&
+                               (in != InType::BF16 || kbytes <= 16384) &&
+                               (in != InType::I8 || long_side == 16 * cus || long_side >= 32 * cus));
     const bool skinny_ok = short_side >= 2 && short_side <= 16 && !gemv_first &&
                            skinny_enabled() && k_fits && (!long_vec || long_ok);
     const bool skinny_long =
@@ -1213,7 +1219,6 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     //    us against 24.7 on the f32 tiles; 2048^3: 109 against 138; 1536 x 167 x 640,
     //    two rounds of blocks: 8 against 16 with small_f32).
     if (in == InType::F32 && !vector_route) {
-        const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
         const int64_t blocks = ((M + 31) / 32) * ((N + 31) / 32);
         const SmallArgs sa{A.p, Bt.p, A.rs, A.ks, Bt.rs, Bt.ks, A.bs, Bt.bs,
                            (int32_t)M, (int32_t)N, (int32_t)k, (int32_t)batch};
@@ -1429,7 +1434,6 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // half the rounds (the same sums: 2 x (2048 x 4096 x 4096) in one round
     // instead of two).
     if (tile == Tile::T128x256w8m16 && batch > 1 && !forced) {
-        const int64_t cus = g_num_cus > 0 ? g_num_cus : 256;
         auto rounds = [&](int64_t bm) {
             return (((M + bm - 1) / bm) * ((N + 255) / 256) * batch + cus - 1) / cus;
         };

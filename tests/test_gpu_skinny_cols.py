@@ -26,7 +26,7 @@ def values(n, dt, seed, dev):
 @pytest.mark.parametrize("shape", [(2, 1024, 17), (3, 1025, 33), (5, 1100, 64), (8, 2048, 1000),
                                    (9, 1536, 129), (16, 1984, 40), (4, 8200, 75), (2, 6144, 300),
                                    (15, 1601, 2050), (2, 16384, 65), (4, 4095, 257), (1, 8300, 70),
-                                   # vectors beyond the LDS: one row group, 8-, 16- and
+                                   # vectors beyond the LDS: one row group, 8-, 24- and
                                    # 32-row ones, K ending inside a step and a chunk,
                                    # more than eight vectors
                                    # i8: both sides of the widths it takes from the
@@ -35,7 +35,9 @@ def values(n, dt, seed, dev):
                                    (1, 1627, 1025), (2, 2528, 4096), (2, 7552, 4097),
                                    (1, 1030, 8), (2, 2048, 9),
                                    (8, 16385, 40), (5, 14008, 2049), (8, 8190, 4100),
-                                   (7, 9300, 8200), (16, 4104, 2048), (12, 5503, 2100)],
+                                   (7, 9300, 8200), (16, 4104, 2048), (12, 5503, 2100),
+                                   # 24- and 32-row groups in one round
+                                   (12, 6100, 4500), (16, 8200, 4500), (9, 8190, 6200)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_unit_row_stride_equals_k_contiguous(dev, dtype, shape):
     m, k, n = shape
