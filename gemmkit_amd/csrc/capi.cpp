@@ -925,12 +925,18 @@ constexpr int64_t kColsMaxRows = 1 << 26;
 //   276, 212), other matrices       0.5 to 0.9
 //   bf16 5 to 16 vectors, short K   1.0 to 1.4    (8 x 512 x 512 times 4096: 530, 375)
 // and below these lines 0.3 to 1.0; small batches gain too little to pay for the pack.
-bool shared_packs(InType in, int64_t nvec, int64_t R, int64_t kbytes, int64_t batch) {
+// Strided vectors, which the in-place kernels have packed and the row kernels stage
+// themselves (slowly when they are many), outweigh a matrix of fewer rows: bf16
+// 2 x 1600 x 24 times 300 33 us, packed 16, 7 x 800 x 24 times 300 24 and 19, but
+// 7 x 800 x 64 no faster, 16 x 800 x 16 21 and 28 and f32 2 x 1600 x 24 30 and 35.
+bool shared_packs(InType in, int64_t nvec, int64_t R, int64_t kbytes, int64_t batch, bool strided) {
     const int64_t outs = batch * R * nvec;
     const bool bf16 = in == InType::BF16;
     if (in == InType::I8) return false;
+    if (strided && nvec <= 8 && kbytes < 4096 && batch * nvec >= (nvec <= 4 ? 4 : 40) * R)
+        return true;
     if (nvec == 1 || !bf16)
-        return (kbytes <= 2048 && outs >= 1 << 17) ||
+        return (kbytes <= 2048 && outs >= (strided ? 1 << 16 : 1 << 17)) ||
                (nvec == 1 && kbytes <= 4096 && outs >= 1 << 19 &&
                 R * kbytes <= (bf16 ? 8 : 5) << 18);
     if (nvec <= 4) return false;
@@ -1130,6 +1136,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // x 4096: 11.5 against 18.9), and reads a row-major matrix in place in any case.
     const Opnd &mat_op = vec_is_a ? Bt : A;
     const int64_t long_side = std::max(M, N), cus = g_num_cus > 0 ? g_num_cus : 256;
+    const Opnd &vec_op = vec_is_a ? A : Bt;
     const bool unit_rows = mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
                            long_side <= kColsMaxRows;
     const bool long_vec = skinny_is_long(in, k, (int)std::min<int64_t>(short_side, 16));
@@ -1149,7 +1156,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     const bool vector_route = skinny_ok || short_side <= 8;
     const bool vec_in_place = skinny_ok && !skinny_long;  // staged from any strides
     const bool shared = unit_rows && batch > 1 && mat_op.bs == 0 &&
-                        shared_packs(in, short_side, long_side, kbytes, batch) &&
+                        shared_packs(in, short_side, long_side, kbytes, batch, vec_op.ks != 1) &&
                         region_fits(rg, pack_bytes(in, long_side, k, batch, mat_op) +
                                             (vec_in_place || (vec_is_a ? a_ok : b_ok)
                                                  ? 0
@@ -1176,7 +1183,6 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
         short_side == 2 ? long_side <= 4096
                         : short_side == 1 && (long_side <= 512 ||
                                               (long_side <= 2048 && (k <= 2048 || k % 128 == 0)));
-    const Opnd &vec_op = vec_is_a ? A : Bt;
     const bool skinny_cols =
         mat_cols && long_side >= kSkinnyColsMinRows &&
         (skinny_ok ||

@@ -99,21 +99,23 @@ def test_batch_and_packed_equal_standalone(dev, dtype):
         assert torch.equal(pk.view(n, m).T.reshape(-1), one)
 
 
-def shared_batch(dev, dtype, batch, m, k, n, ws):
-    """A batch on one row-major matrix (zero batch stride), strided in C."""
+def shared_batch(dev, dtype, batch, m, k, n, ws, strided=False):
+    """A batch on one row-major matrix (zero batch stride), strided in C (and A:
+    vectors side by side)."""
     dt = DT[dtype]
     a, b = values(batch * m * k, dt, 7, dev), values(k * n, dt, 8, dev)
+    rsa, csa = (1, m) if strided else (k, 1)
     cbs = m * n + 5
     c = torch.zeros(batch * cbs, dtype=dt, device=dev)
 
     def call(ws=ws):
-        gk.gemm_batched_unchecked(batch, m, k, n, 1.0, a, k, 1, m * k, b, n, 1, 0, 0.0, c, n, 1,
-                                  cbs, ws=ws)
+        gk.gemm_batched_unchecked(batch, m, k, n, 1.0, a, rsa, csa, m * k, b, n, 1, 0, 0.0, c, n,
+                                  1, cbs, ws=ws)
 
     def check():
         for z in (0, 1, batch // 2, batch - 2, batch - 1):
             one = torch.zeros(m * n, dtype=dt, device=dev)
-            gk.gemm_unchecked(m, k, n, 1.0, a, k, 1, b, n, 1, 0.0, one, n, 1, a_off=z * m * k)
+            gk.gemm_unchecked(m, k, n, 1.0, a, rsa, csa, b, n, 1, 0.0, one, n, 1, a_off=z * m * k)
             assert torch.equal(c[z * cbs:z * cbs + m * n], one), z
         assert (c.view(batch, cbs)[:, m * n:] == 0).all()
 
@@ -134,18 +136,21 @@ def test_shared_matrix_bounded_workspace(dev, dtype, batch, m, k, n):
     check()
 
 
-@pytest.mark.parametrize("dtype,batch,m,k,n", [
-    ("f32", 300, 1, 256, 500), ("f32", 150, 3, 500, 333), ("f32", 40, 9, 300, 400),
-    ("bf16", 300, 1, 700, 500), ("bf16", 600, 7, 600, 260), ("bf16", 100, 13, 800, 400)])
-def test_shared_matrix_of_short_rows_is_packed(dev, dtype, batch, m, k, n):
+@pytest.mark.parametrize("dtype,batch,m,k,n,strided", [
+    ("f32", 300, 1, 256, 500, False), ("f32", 150, 3, 500, 333, False),
+    ("f32", 40, 9, 300, 400, False), ("bf16", 300, 1, 700, 500, False),
+    ("bf16", 600, 7, 600, 260, False), ("bf16", 100, 13, 800, 400, False),
+    ("bf16", 300, 2, 1600, 24, True), ("f32", 300, 7, 900, 33, True), ("f32", 300, 16, 256, 16, True)])
+def test_shared_matrix_of_short_rows_is_packed(dev, dtype, batch, m, k, n, strided):
     """One pack serves the batch; under capture, where the workspace cannot grow, one
     vector's matrix is read in place: the same bits every way."""
     ws = gk.Workspace()
-    call, check, c = shared_batch(dev, dtype, batch, m, k, n, ws)
+    call, check, c = shared_batch(dev, dtype, batch, m, k, n, ws, strided)
     call()
     pad = 16 // DT[dtype].itemsize
     assert ws.bytes() >= n * (k + pad - 1) // pad * pad * DT[dtype].itemsize
-    assert ws.bytes() < 8 * batch * m * n * 4 or m == 1
+    # (partial sums, or packed vectors, would take more)
+    assert ws.bytes() < 8 * batch * m * n * 4 + strided * batch * m * k or m == 1
     check()
     # captured: with the arena of that call, and one vector with none
     for arena in (ws, gk.Workspace()):
