@@ -1177,7 +1177,7 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // two vectors on it 9.9 us, one on the GEMV 16.2), and narrow matrices, which
     // leave the GEMV few workgroups (packed first, GEMV, skinny: 1 x 2048 x 179 6.6,
     // 10.0, 5.1 us; 2 x 7552 x 64 7.2, 11.1, 5.7; 2 x 4096 x 4096 21.7, 11.3, 8.3; 1 x
-    // 1440 x 1305 8.6, 10.3, 7.2; but 1 x 2528 x 2048 11.9, 7.8, 9.1, 1 x 2528 x 4096
+    // 1440 x 1305 8.5, 10.4, 8.1; but 1 x 2528 x 2048 11.9, 7.8, 9.1, 1 x 2528 x 4096
     // 16.6, 8.4, 9.7 and 2 x 4096 x 8000 34, 12.9, 14.4) while its partial sums have room.
     const bool i8_narrow =
         short_side == 2 ? long_side <= 4096

@@ -23,11 +23,12 @@
 // small.hip would serve, whose sixteen partial sums round less) the small sum
 // runs over all of K and is added once.  With ml and lm left out too, together up
 // to 2^-24, and all products in one sum a single term erred by up to 1.4 ulp
-// (2048^3: 95 us instead of 112).
-// Measured (row-major, against the f32 tiles with B packed first): 2048^3 112 us =
-// 153 TFLOP/s against 138, relative error on normal inputs 2.1e-7 against 8.1e-7;
-// 1024^3 22.7 against 29.2, 1.5e-7 against 5.7e-7; 488 x 3136 x 2512 78 against 95.
-// Bound by the matrix cores at the clock the chip's power limit leaves them.
+// (2048^3: 93 us instead of 108).
+// Measured (row-major, against the f32 tiles with B packed first): 2048^3 108 us =
+// 159 TFLOP/s against 138, relative error on normal inputs 2.1e-7 against 8.1e-7;
+// 1024^3 22.5 against 29.2, 1.5e-7 against 5.7e-7; 488 x 2512 x 3136 76 against 95.
+// Bound by the matrix cores at the clock the chip's power limit leaves them: 1270
+// TFLOP/s of bf16 products, where library products reach 1338 (4096^3) to 1610.
 //
 // Range.  Elements are scaled by 2^23 as they are split and the sums by 2^-46 at
 // the end, both exact (a subnormal result is rounded once more): every part of
@@ -54,11 +55,12 @@
 // stage n left, and issues the loads of stage n+5; then a barrier, and the roles
 // change.  The matrix cores so always have a wave with nothing else to wait
 // for, and the splitting, the LDS traffic and the memory latency run beside it.
-// (All eight waves doing all of it in turn: 102 us on 2048^3 against 85.)  A K that
-// is no multiple of 32 has its short stage first, outside the loop.
+// (All eight waves doing all of it in turn, with six products: 102 us on 2048^3
+// against 85.)  A K that is no multiple of 32 has its short stage first, outside
+// the loop.
 //
-// Operands are read in place with any strides (no pack): a k-contiguous operand
-// as two 16-byte loads of 8 k of a row per thread, any other as 8 element loads
+// Operands are read in place with any strides (the caller packs those that this
+// would read a cache line at a time): a k-contiguous operand as two 16-byte loads of 8 k of a row per thread, any other as 8 element loads
 // with the lanes along the rows (coalesced when the rows are contiguous).
 // LDS holds, per stage and part, 64-byte rows of 32 k; row r keeps its 16-byte
 // chunk c in slot c ^ ((r >> 2) & 3), which spreads 16 consecutive rows (a
@@ -475,9 +477,11 @@ hipError_t launch_f32x(const SmallArgs &g, const EpiParams &ep, bool fine, int c
         ep.kind != EpiKind::F32)
         return hipErrorInvalidValue;
     // 128 x 128 tiles, one per CU, against 64 x 64 ones, two per CU at a time: a round
-    // of large tiles takes about 3.2 times a round of small ones (2048^3: 86 us in
-    // one round against 114 in four; 2048 x 2049 x 2048, whose 272 large tiles take
-    // two rounds: 175 against 145; 1024^3, a quarter of the CUs: 46 against 22).
+    // of large tiles takes about 3 times a round of small ones (2048^3: 110 us in
+    // one round against 142 in four; 1536 x 1000 x 1536 50 in one against 53 in three;
+    // 3000 x 2000 x 3000 285 in three against 298 in nine; 2048 x 2048 x 2049, whose 272
+    // large tiles take two rounds: 185 against 161 in five; 1024^3, a quarter of the
+    // CUs: 46 against 22).
     const int64_t c = cus > 0 ? cus : 256;
     auto rounds = [&](int64_t t) {
         return (((g.M + t - 1) / t) * ((g.N + t - 1) / t) * g.batch + c - 1) / c;
@@ -488,7 +492,7 @@ hipError_t launch_f32x(const SmallArgs &g, const EpiParams &ep, bool fine, int c
     if (fine)
         return rounds(64) == 1 ? f32x_go<64, 64, true, 2>(g, ep, stream)
                                : f32x_go<64, 64, true, 4>(g, ep, stream);
-    if (16 * rounds(128) <= 5 * rounds(64))
+    if (3 * rounds(128) <= rounds(64))
         return f32x_go<128, 128, false, 2>(g, ep, stream);
     return f32x_go<64, 64, false, 4>(g, ep, stream);
 }
