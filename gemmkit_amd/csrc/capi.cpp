@@ -1130,22 +1130,31 @@ int run_fit(const Region &rg, InType in, EpiParams ep, int64_t m, int64_t k, int
     // and two rounds of 16-row items it gains little or loses to them (bf16 16 x 8000:
     // 4500 rows 19.9 us against 17.0, 5810 21.0 against 20.1, 7000 24.7 against 22.8, i8
     // 16 x 16384 alike): a k-contiguous i8 matrix, whose sums have no order, stays on
-    // the tiles there; float ones must sum alike whatever their strides, and a row-major
-    // matrix, read in place, gains far more.  i8 takes skinny_long with
-    // 5..8 vectors already where the LDS would hold one workgroup a CU (8 x 11008
-    // x 4096: 11.5 against 18.9), and reads a row-major matrix in place in any case.
+    // the tiles there while the workspace has room for their sums; float ones must sum
+    // alike whatever their strides, and a row-major matrix, read in place, gains far
+    // more.  i8 takes skinny_long with 5..8 vectors already where the LDS would hold one
+    // workgroup a CU (8 x 11008 x 4096: 11.5 against 18.9), and reads a row-major matrix
+    // in place in any case.
     const Opnd &mat_op = vec_is_a ? Bt : A;
     const int64_t long_side = std::max(M, N), cus = g_num_cus > 0 ? g_num_cus : 256;
     const Opnd &vec_op = vec_is_a ? A : Bt;
     const bool unit_rows = mat_op.rs == 1 && mat_op.ks != 1 && kbytes >= kGemvColsMinBytes &&
                            long_side <= kColsMaxRows;
     const bool long_vec = skinny_is_long(in, k, (int)std::min<int64_t>(short_side, 16));
+    // (the tiles' partial sums and packs, which skinny_long does without)
+    auto tiles_fit = [&] {
+        const int64_t slabs = choose_splits(M, N, k, esz) * M * N * 4 * batch;
+        return region_fits(rg, (size_t)round_up64(std::min(slabs, kSlabMax), 256) +
+                                   (a_ok ? 0 : pack_bytes(in, M, k, batch, A)) +
+                                   (b_ok ? 0 : pack_bytes(in, N, k, batch, Bt)));
+    };
     const bool long_ok =
         short_side <= 8 ? short_side > (in == InType::BF16 ? 2 : kGemvColsMaxVec)
                         : (in == InType::I8 && unit_rows) ||
                               (long_side >= 16 * cus &&
                                (in != InType::BF16 || kbytes <= 16384) &&
-                               (in != InType::I8 || long_side == 16 * cus || long_side >= 32 * cus));
+                               (in != InType::I8 || long_side == 16 * cus ||
+                                long_side >= 32 * cus || !tiles_fit()));
     const bool skinny_ok = short_side >= 2 && short_side <= 16 && !gemv_first &&
                            skinny_enabled() && k_fits && (!long_vec || long_ok);
     const bool skinny_long =

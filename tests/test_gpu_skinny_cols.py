@@ -173,6 +173,37 @@ def test_shared_matrix_of_short_rows_is_packed(dev, dtype, batch, m, k, n, strid
             check()
 
 
+@pytest.mark.parametrize("m,k,n,layout", [(16, 8208, 4500, "col"), (2, 2048, 300, "row")])
+def test_i8_routes_without_workspace(dev, m, k, n, layout):
+    """i8 takes the faster of two routes only while its partial sums have room: under
+    capture with an empty arena that cannot grow, the one without any."""
+    a, w = values(m * k, torch.int8, 9, dev), values(k * n, torch.int8, 10, dev)
+    rsb, csb = (1, k) if layout == "col" else (n, 1)
+    c = torch.zeros(m * n, dtype=torch.int32, device=dev)
+
+    def call(ws):
+        gk.gemm_i8_unchecked(m, k, n, 1, a, k, 1, w, rsb, csb, 0, c, n, 1, ws=ws)
+
+    call(gk.Workspace())
+    want = (a.view(m, k).double() @ torch.as_strided(w, (k, n), (rsb, csb)).double()).reshape(-1)
+    assert torch.equal(c.double(), want)
+    ws = gk.Workspace()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    gk.set_synchronous(False)
+    try:
+        with torch.cuda.graph(graph):
+            call(ws)
+    finally:
+        gk.set_synchronous(True)
+    assert ws.bytes() == 0
+    for _ in range(3):
+        c.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c.double(), want)
+
+
 def test_nonfinite_columns_stay_apart(dev):
     """A row of infinities or NaN reaches its own outputs only, past K neither."""
     m, k, n = 3, 1030, 50
