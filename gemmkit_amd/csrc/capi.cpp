@@ -828,7 +828,11 @@ constexpr int64_t kF32xMinK = 128;
 // Whether an f32 product runs on the bf16 matrix cores (f32x.hip), given its K
 // ranges on the tiles otherwise: K of 128 or more (below that its four or fewer
 // stages do not pay for its start: 951 x 104 x 2368 with k-contiguous operands 15.7
-// us against 13.9 on the f32 tiles), and no split, or more than one round of the
+// us against 13.9 on the f32 tiles; with both operands k-contiguous and aligned the
+// tiles, which then need no pack, stay ahead up to K of about 400, 3488 x 208 x 253 7.5
+// against 9.4, 1000 x 300 x 1000 9.5 against 10.5, 1500 x 700 x 1500 48 against 39, but
+// sums must be alike whatever the strides, and row-major those are 14.4 against 10.8
+// and 56 against 39), and no split, or more than one round of the
 // 32 x 32 blocks of small_f32 while its waves' shares are short (two rounds, 1500 x K x
 // 300: 9.6 us against 16.5 at K = 320, 20 against 25 at 1024, 66 against 89 at 4096;
 // K of 385 to 512, one group of loads for each of small_f32's waves, 11.5 to 12.4

@@ -60,8 +60,9 @@
 // the loop.
 //
 // Operands are read in place with any strides (the caller packs those that this
-// would read a cache line at a time): a k-contiguous operand as two 16-byte loads of 8 k of a row per thread, any other as 8 element loads
-// with the lanes along the rows (coalesced when the rows are contiguous).
+// would read a cache line at a time): a k-contiguous operand as two 16-byte loads
+// of 8 k of a row per thread, any other as 8 element loads with the lanes along the
+// rows (coalesced when the rows are contiguous).
 // LDS holds, per stage and part, 64-byte rows of 32 k; row r keeps its 16-byte
 // chunk c in slot c ^ ((r >> 2) & 3), which spreads 16 consecutive rows (a
 // fragment read, and the writes of either load form) over distinct banks.
